@@ -527,7 +527,7 @@ int dem_instance_observables_noalloc(dem_ctx *ctx, double *out);
  * usual.  The results are bitwise those of stepping without the graph. */
 int dem_use_graph(dem_ctx *ctx, int on);
 /* Autotuner: times the contact pass on the current state for every shape
- * (lane groups of 1..16 lanes per particle, contact-queue tiles of 8..64
+ * (lane groups of 1..16 lanes per particle, tiles of 8, 16, 32 or 64
  * particles per wave, given as -8..-64) and block size (64..256), in the
  * form the steps run (with the integrator when the pass integrates), and
  * keeps the fastest for this context.  State and history are left

@@ -32,7 +32,9 @@ __global__ void __launch_bounds__(kBlock) k_adj_mask(AdjMaskArgs a)
     const int i = blockIdx.x * kBlock + threadIdx.x;
     if (i >= a.n) return;
     const double4 pi = a.xr[i];
-    for (int e = a.nstart[i]; e < a.nstart[i + 1]; e++) {
+    const Row row = list_row(a.nstart, a.n, i);
+    for (int q = 0; q < row.cnt; q++) {
+        const int e = row.entry(q);
         const uint32_t w = a.nj[e];
         const int j = (int)(w & kJMask);
         const int code = (int)((w >> 26) & 31u);
@@ -59,12 +61,16 @@ __global__ void __launch_bounds__(kBlock) k_adj_rev(const int *nstart, const uin
 {
     const int i = blockIdx.x * kBlock + threadIdx.x;
     if (i >= n) return;
-    for (int e = nstart[i]; e < nstart[i + 1]; e++) {
+    const Row row = list_row(nstart, n, i);
+    for (int k = 0; k < row.cnt; k++) {
+        const int e = row.entry(k);
         const uint32_t w = nj[e];
         const int j = (int)(w & kJMask);
         const int mirror = 26 - (int)((w >> 26) & 31u);
         int r = -1;
-        for (int f = nstart[j]; f < nstart[j + 1]; f++) {
+        const Row rj = list_row(nstart, n, j);
+        for (int q = 0; q < rj.cnt; q++) {
+            const int f = rj.entry(q);
             const uint32_t u = nj[f];
             if ((int)(u & kJMask) == i && (int)((u >> 26) & 31u) == mirror) {
                 r = f;
@@ -104,7 +110,9 @@ __global__ void __launch_bounds__(kBlock) k_adj_step(AdjArgs a)
     double ax[3] = {0, 0, 0}, av[3] = {0, 0, 0}, aw[3] = {0, 0, 0};
     LawP gq{0, 0, 0, 0};
     const int dn = a.dnum;
-    for (int e = a.nstart[i]; e < a.nstart[i + 1]; e++) {
+    const Row row = list_row(a.nstart, a.n, i);
+    for (int q = 0; q < row.cnt; q++) {
+        const int e = row.entry(q);
         const uint32_t w = a.nj[e];
         const int j = (int)(w & kJMask);
         const int code = (int)((w >> 26) & 31u);

@@ -308,7 +308,9 @@ __global__ void __launch_bounds__(kBlock) k_bond(BondArgs a)
     const double xi[3] = {pi.x, pi.y, pi.z};
     const double vi[3] = {vmi.x, vmi.y, vmi.z};
     const double omi[3] = {wi.x, wi.y, wi.z};
-    for (int e = a.nstart[i]; e < a.nstart[i + 1]; e++) {
+    const Row row = list_row(a.nstart, a.n, i);
+    for (int k = 0; k < row.cnt; k++) {
+        const int e = row.entry(k);
         const uint32_t w = a.nj[e];
         const int j = (int)(w & kJMask);
         const int code = (int)((w >> 26) & 31u);
@@ -385,19 +387,24 @@ __global__ void __launch_bounds__(kBlock) k_bond_rev(const int *nstart, const ui
 {
     const int i = blockIdx.x * kBlock + threadIdx.x;
     if (i >= n) return;
-    for (int e = nstart[i]; e < nstart[i + 1]; e++) {
+    const Row row = list_row(nstart, n, i);
+    for (int k = 0; k < row.cnt; k++) {
+        const int e = row.entry(k);
         const uint32_t w = nj[e];
         const int j = (int)(w & kJMask);
         const int code = (int)((w >> 26) & 31u);
         int r = -1;
-        if (code == kNoShift)
-            for (int f = nstart[j]; f < nstart[j + 1]; f++) {
+        if (code == kNoShift) {
+            const Row rj = list_row(nstart, n, j);
+            for (int q = 0; q < rj.cnt; q++) {
+                const int f = rj.entry(q);
                 const uint32_t u = nj[f];
                 if ((int)(u & kJMask) == i && (int)((u >> 26) & 31u) == kNoShift) {
                     r = f;
                     break;
                 }
             }
+        }
         rev[e] = r;
     }
 }

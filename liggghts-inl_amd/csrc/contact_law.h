@@ -185,7 +185,9 @@ __host__ __device__ constexpr int chain_max_dnum(int nm) { return chain_off_shea
 // CH: a cohesion model sits between the normal and tangential models; coh =
 // its force and torque on this side, cmode CM_BOND adds them to the chain,
 // CM_BOND_NONLINEAR replaces the normal force with them, CM_OFF skips.
-template <int NM, bool CH = false>
+// RH: whether the chain keeps a rolling history, 0 or 1 where the caller's
+// history layout says so at compile time, -1 to ask the model.
+template <int NM, bool CH = false, int RH = -1>
 __device__ inline void contact_fp64(const Model &M, const Layout &L, const double *mat, const ContactIn &c,
                                     double *h, bool update, double F[3], double T[3],
                                     const double *coh = nullptr, int cmode = CM_OFF)
@@ -316,7 +318,7 @@ __device__ inline void contact_fp64(const Model &M, const Layout &L, const doubl
     }
 
     // ---- rolling friction
-    if (M.rolling && L.off_roll >= 0) {
+    if (RH == 1 || (RH < 0 && M.rolling && L.off_roll >= 0)) {
         double w1, w2, w3, r_inertia;
         if (c.is_wall) {
             w1 = wr1; w2 = wr2; w3 = wr3;
@@ -417,11 +419,13 @@ __device__ inline bool contact_close(const Layout &L, double *hp)
 
 // Mixed precision: the overlap deltan (a small difference of large numbers)
 // and the history integration are FP64; everything else of the law is FP32.
-// Hertz chains only (shear at slot 0, rolling torque at slot 3).
+// Hertz chains only (shear at slot 0, rolling torque at slot 3).  Every fused
+// multiply-add is written out: left to the compiler, which of two products is
+// fused depends on the kernel around the law, and two kernels would round the
+// same contact differently.
 __device__ inline void contact_mixed(const Model &M, const double *mat, const ContactIn &c,
                                      double *h, bool update, double F[3], double T[3])
 {
-#pragma clang fp contract(fast)
     const float SQRT_FIVE_OVER_SIX = 0.912870929175276856f;
     const float rinv = (float)c.rinv;
     const float enx = (float)c.delta[0] * rinv;
@@ -431,8 +435,8 @@ __device__ inline void contact_mixed(const Model &M, const double *mat, const Co
     const float vr1 = (float)(c.vi[0] - c.vj[0]);
     const float vr2 = (float)(c.vi[1] - c.vj[1]);
     const float vr3 = (float)(c.vi[2] - c.vj[2]);
-    const float vn = vr1 * enx + vr2 * eny + vr3 * enz;
-    const float vt1 = vr1 - vn * enx, vt2 = vr2 - vn * eny, vt3 = vr3 - vn * enz;
+    const float vn = fmaf(vr3, enz, fmaf(vr1, enx, vr2 * eny));
+    const float vt1 = fmaf(-enx, vn, vr1), vt2 = fmaf(-eny, vn, vr2), vt3 = fmaf(-enz, vn, vr3);
     const double deltan_d = c.radsum - c.r;
     const float deltan = (float)deltan_d;
     const float dx = (float)c.delta[0], dy = (float)c.delta[1], dz = (float)c.delta[2];
@@ -446,13 +450,13 @@ __device__ inline void contact_mixed(const Model &M, const double *mat, const Co
     } else {
         cri = (float)(c.radi - 0.5 * deltan_d);
         const float crj = (float)(c.radj - 0.5 * deltan_d);
-        wr1 = (cri * (float)c.wi[0] + crj * (float)c.wj[0]) * rinv;
-        wr2 = (cri * (float)c.wi[1] + crj * (float)c.wj[1]) * rinv;
-        wr3 = (cri * (float)c.wi[2] + crj * (float)c.wj[2]) * rinv;
+        wr1 = fmaf((float)c.wi[0], cri, crj * (float)c.wj[0]) * rinv;
+        wr2 = fmaf((float)c.wi[1], cri, crj * (float)c.wj[1]) * rinv;
+        wr3 = fmaf((float)c.wi[2], cri, crj * (float)c.wj[2]) * rinv;
     }
-    const float vtr1 = vt1 - (dz * wr2 - dy * wr3);
-    const float vtr2 = vt2 - (dx * wr3 - dz * wr1);
-    const float vtr3 = vt3 - (dy * wr1 - dx * wr2);
+    const float vtr1 = vt1 - fmaf(wr2, dz, -(wr3 * dy));
+    const float vtr2 = vt2 - fmaf(wr3, dx, -(wr1 * dz));
+    const float vtr3 = vt3 - fmaf(wr1, dy, -(wr2 * dx));
 
     const int it = c.itype, jt = c.jtype;
     const float radi = (float)c.radi, radj = (float)c.radj;
@@ -468,22 +472,24 @@ __device__ inline void contact_mixed(const Model &M, const double *mat, const Co
     const float kt = St;
     const float gamman = -2.f * SQRT_FIVE_OVER_SIX * beta * sqrtf(Sn * meff);
     const float gammat = M.tdamp ? -2.f * SQRT_FIVE_OVER_SIX * beta * sqrtf(St * meff) : 0.f;
-    float Fn = -gamman * vn + kn * deltan;
+    float Fn = fmaf(kn, deltan, -(gamman * vn));
     if ((c.is_wall ? M.lw.limitf : M.lp.limitf) && (Fn < 0.f)) Fn = 0.f;
 
     double *shear = h;
     if (update) {
         const double dt = M.dt;
-        shear[0] += (double)vtr1 * dt;
-        shear[1] += (double)vtr2 * dt;
-        shear[2] += (double)vtr3 * dt;
-        const double rsht = shear[0] * enx + shear[1] * eny + shear[2] * enz;
-        shear[0] -= rsht * enx;
-        shear[1] -= rsht * eny;
-        shear[2] -= rsht * enz;
+        shear[0] = fma((double)vtr1, dt, shear[0]);
+        shear[1] = fma((double)vtr2, dt, shear[1]);
+        shear[2] = fma((double)vtr3, dt, shear[2]);
+        const double rsht = fma(shear[2], (double)enz, fma(shear[0], (double)enx, shear[1] * (double)eny));
+        shear[0] = fma(-rsht, (double)enx, shear[0]);
+        shear[1] = fma(-rsht, (double)eny, shear[1]);
+        shear[2] = fma(-rsht, (double)enz, shear[2]);
     }
     const float s0 = (float)shear[0], s1 = (float)shear[1], s2 = (float)shear[2];
-    const float shrmag = sqrtf(s0 * s0 + s1 * s1 + s2 * s2);
+    // (planes and pairs keep the orders their results have always had)
+    const float s01 = c.is_wall ? fmaf(s0, s0, s1 * s1) : fmaf(s1, s1, s0 * s0);
+    const float shrmag = sqrtf(fmaf(s2, s2, s01));
     const float xmu = (float)tbl(mat, M_MU, it, jt);
     float Ft1 = -(kt * s0), Ft2 = -(kt * s1), Ft3 = -(kt * s2);
     const float Ft_shear = kt * shrmag;
@@ -502,16 +508,16 @@ __device__ inline void contact_mixed(const Model &M, const double *mat, const Co
             Ft1 = Ft2 = Ft3 = 0.f;
         }
     } else {
-        Ft1 -= gammat * vtr1;
-        Ft2 -= gammat * vtr2;
-        Ft3 -= gammat * vtr3;
+        Ft1 = fmaf(-gammat, vtr1, Ft1);
+        Ft2 = fmaf(-gammat, vtr2, Ft2);
+        Ft3 = fmaf(-gammat, vtr3, Ft3);
     }
-    const float tor1 = eny * Ft3 - enz * Ft2;
-    const float tor2 = enz * Ft1 - enx * Ft3;
-    const float tor3 = enx * Ft2 - eny * Ft1;
-    F[0] = (double)(Fn * enx + Ft1);
-    F[1] = (double)(Fn * eny + Ft2);
-    F[2] = (double)(Fn * enz + Ft3);
+    const float tor1 = fmaf(eny, Ft3, -(enz * Ft2));
+    const float tor2 = fmaf(enz, Ft1, -(enx * Ft3));
+    const float tor3 = fmaf(enx, Ft2, -(eny * Ft1));
+    F[0] = (double)fmaf(Fn, enx, Ft1);
+    F[1] = (double)fmaf(Fn, eny, Ft2);
+    F[2] = (double)fmaf(Fn, enz, Ft3);
     float T0 = -cri * tor1, T1 = -cri * tor2, T2 = -cri * tor3;
 
     if (M.rolling) {
@@ -525,14 +531,14 @@ __device__ inline void contact_mixed(const Model &M, const double *mat, const Co
             w3 = (float)(c.wi[2] - c.wj[2]);
             const float ri = (float)c.mi * radi * radi;
             const float rj = (float)c.mj * radj * radj;
-            r_inertia = 1.4f * ri * rj / (ri + rj);
+            r_inertia = 1.4f * ri * rj / fmaf((float)c.mj * radj, radj, ri);
         }
         float wt0, wt1, wt2;
         if (M.torsion) {
             wt0 = w1; wt1 = w2; wt2 = w3;
         } else {
-            const float wdd = w1 * enx + w2 * eny + w3 * enz;
-            wt0 = w1 - enx * wdd; wt1 = w2 - eny * wdd; wt2 = w3 - enz * wdd;
+            const float wdd = fmaf(w3, enz, fmaf(w1, enx, w2 * eny));
+            wt0 = fmaf(-enx, wdd, w1); wt1 = fmaf(-eny, wdd, w2); wt2 = fmaf(-enz, wdd, w3);
         }
         const float rmu = (float)tbl(mat, M_MUR, it, jt);
         float kr;
@@ -541,10 +547,10 @@ __device__ inline void contact_mixed(const Model &M, const double *mat, const Co
         else kr = (float)M.krs * kn * rmu * rmu * reff * reff;
         const double dtkr = M.dt * (double)kr;
         double *ch = h + 3;
-        double rt0 = ch[0] + dtkr * wt0;
-        double rt1 = ch[1] + dtkr * wt1;
-        double rt2 = ch[2] + dtkr * wt2;
-        const float mag = sqrtf((float)(rt0 * rt0 + rt1 * rt1 + rt2 * rt2));
+        double rt0 = fma(dtkr, (double)wt0, ch[0]);
+        double rt1 = fma(dtkr, (double)wt1, ch[1]);
+        double rt2 = fma(dtkr, (double)wt2, ch[2]);
+        const float mag = sqrtf((float)fma(rt2, rt2, fma(rt0, rt0, rt1 * rt1)));
         const float rmax = fabsf(Fn) * reff * rmu;
         if (mag > rmax) {
             const double factor = (double)(rmax / mag);

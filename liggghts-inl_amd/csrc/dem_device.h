@@ -7,9 +7,13 @@
 //   f4  double4  (fx, fy, fz, -)             32 B
 //   t4  double4  (tx, ty, tz, -)             32 B
 //   tag int, orig int (upload position), img int4 (periodic image counts)
-// Neighbour list: full (both directions), CSR rows per particle:
-//   nstart[n+1]; nj[e] = j | bond << 25 | shift << 26 | flag << 31; hist[e*dnum + k]
-//   (history slots: hysteretic 12, shear 3, rolling 3, cohesion 14/28)
+// Neighbour list: full (both directions), each particle's row in two parts:
+//   nstart[2n+1]: the partners that touched at the build, entries
+//   [nstart[i], nstart[i+1]), then the others, [nstart[n+i], nstart[n+i+1]);
+//   nj[e] = j | bond << 25 | shift << 26 | flag << 31; hist[e*dnum + k]
+//   (history slots: hysteretic 12, shear 3, rolling 3, cohesion 14/28).
+//   The touching entries of all particles come first, so the histories that
+//   a step reads and writes fill whole cache lines.
 // Primitive walls: wmask[i] bit k = atom in wall k's list; whist[(i*np+k)*dnum]
 // Mesh walls, per mesh: TriGeo records; per particle a CSR row (mstart) of
 // candidate triangles (mcand, ascending id) and as many contact slots
@@ -149,6 +153,21 @@ struct Grid {
     int maxc;
     int reach;           // cells per cutneighmax: the stencil is 2*reach+1 cells wide
 };
+
+// One particle's row: entry k of it, touching partners first.
+struct Row {
+    int a0, na, b0, cnt;
+    __host__ __device__ int entry(int k) const { return k < na ? a0 + k : b0 + (k - na); }
+};
+__host__ __device__ inline Row list_row(const int *nstart, int n, int i)
+{
+    Row r;
+    r.a0 = nstart[i];
+    r.na = nstart[i + 1] - r.a0;
+    r.b0 = nstart[n + i];
+    r.cnt = r.na + nstart[n + i + 1] - r.b0;
+    return r;
+}
 
 __host__ __device__ inline void shift_decode(int code, int &sx, int &sy, int &sz)
 {

@@ -154,7 +154,7 @@ struct dem_ctx {
 
     // neighbour list, double buffered for the history remap
     int lcur = 0;
-    int *nstart[2] = {};
+    int *nstart[2] = {};     // 2 n + 1 row starts (dem_device.h)
     uint32_t *nj[2] = {};
     double *hist[2] = {};
     int64_t ecap[2] = {0, 0};
@@ -898,7 +898,7 @@ static int setup_grid(dem_ctx *ctx)
             return DEM_ERR_HIP;
         ctx->nkeys_cap = G.nkeys + 1;
     }
-    const int need = std::max(scan_tmp_size(G.nkeys + 1), scan_tmp_size(ctx->n + 1));
+    const int need = std::max(scan_tmp_size(G.nkeys + 1), scan_tmp_size(2 * ctx->n + 1));
     if (need > ctx->scan_tmp_cap) {
         if (dev_alloc(ctx, &ctx->scan_tmp, need)) return DEM_ERR_HIP;
         ctx->scan_tmp_cap = need;
@@ -942,7 +942,7 @@ extern "C" int dem_upload_state(dem_ctx *ctx, int n, const double *x, const doub
                 || dev_alloc(ctx, &ctx->wt[b], c) || dev_alloc(ctx, &ctx->tag[b], c)
                 || dev_alloc(ctx, &ctx->orig[b], c) || dev_alloc(ctx, &ctx->img[b], c)
                 || dev_alloc(ctx, &ctx->whist[b], c * std::max(wdn, 1))
-                || dev_alloc(ctx, &ctx->nstart[b], c + 1) || dev_alloc(ctx, &ctx->gmask[b], c))
+                || dev_alloc(ctx, &ctx->nstart[b], 2 * c + 1) || dev_alloc(ctx, &ctx->gmask[b], c))
                 return DEM_ERR_HIP;
         }
         if (dev_alloc(ctx, &ctx->f4, c) || dev_alloc(ctx, &ctx->t4, c) || dev_alloc(ctx, &ctx->xhold, c)
@@ -1048,7 +1048,7 @@ static int mesh_rebuild(dem_ctx *ctx, MeshDev &m, bool captured = false)
     launch_fill_int(m.mstart[b] + n, 0, 1, s);
     launch_fill_int(ctx->d_small + 3, 0, 1, s);
     launch_mesh_stage(na, s);   // one search: counts and staged rows
-    launch_row_max(m.mstart[b], n, ctx->d_small + 3, s);
+    launch_row_max(m.mstart[b], n, 1, ctx->d_small + 3, s);
     launch_scan(m.mstart[b], n + 1, ctx->scan_tmp, s);
     KCHK();
     const int dw = ctx->M.wdnum;
@@ -1206,22 +1206,22 @@ static int rebuild(dem_ctx *ctx, bool captured = false)
     na.stage = ctx->stage;
     const bool staged = neigh_staged();
     launch_fill_int(ctx->d_small + 1, 0, 1, s);
-    launch_fill_int(ctx->nstart[l1] + n, 0, 1, s);
+    launch_fill_int(ctx->nstart[l1] + 2 * n, 0, 1, s);
     if (staged) launch_neigh_stage(na, s);
     else launch_neigh_count(na, s);
     KCHK();
-    launch_scan(ctx->nstart[l1], n + 1, ctx->scan_tmp, s);
+    launch_scan(ctx->nstart[l1], 2 * n + 1, ctx->scan_tmp, s);
     KCHK();
     int hsmall[2] = {0, 0};
     if (!captured) {
-        HIPCHK(hipMemcpyAsync(&hsmall[0], ctx->nstart[l1] + n, sizeof(int), hipMemcpyDeviceToHost, s));
+        HIPCHK(hipMemcpyAsync(&hsmall[0], ctx->nstart[l1] + 2 * n, sizeof(int), hipMemcpyDeviceToHost, s));
         HIPCHK(hipMemcpyAsync(&hsmall[1], ctx->d_small + 1, sizeof(int), hipMemcpyDeviceToHost, s));
         HIPCHK(hipStreamSynchronize(s));
         if (hsmall[1] > ctx->p.neigh_one)
             return fail(ctx, DEM_ERR_OVERFLOW, "Neighbor list overflow, boost neigh_modify one");
         if (ensure_list_cap(ctx, l1, hsmall[0])) return DEM_ERR_NOMEM;
     }
-    if (captured) launch_cap_guard(ctx->nstart[l1], n, ctx->ecap[l1], ctx->d_small + 4, ctx->d_small, 8, s);
+    if (captured) launch_cap_guard(ctx->nstart[l1], 2 * n, ctx->ecap[l1], ctx->d_small + 4, ctx->d_small, 8, s);
     na.ecap = ctx->ecap[l1];
     na.coh_off = ctx->M.cohesion != CM_OFF ? ctx->M.lp.off_coh : -1;
     na.err = ctx->d_small;
@@ -1668,7 +1668,7 @@ static int grow_particles(dem_ctx *ctx, int c)
             || dev_grow(ctx, &ctx->wt[b], oc, nc) || dev_grow(ctx, &ctx->tag[b], oc, nc)
             || dev_grow(ctx, &ctx->orig[b], oc, nc) || dev_grow(ctx, &ctx->img[b], oc, nc)
             || dev_grow(ctx, &ctx->whist[b], oc * wdn, nc * wdn)
-            || dev_grow(ctx, &ctx->nstart[b], oc ? oc + 1 : 0, nc + 1) || dev_grow(ctx, &ctx->gmask[b], oc, nc))
+            || dev_grow(ctx, &ctx->nstart[b], oc ? 2 * oc + 1 : 0, 2 * nc + 1) || dev_grow(ctx, &ctx->gmask[b], oc, nc))
             return DEM_ERR_HIP;
         if (ctx->xo[b] && dev_grow(ctx, &ctx->xo[b], oc, nc)) return DEM_ERR_HIP;
         if (ctx->brid[b] && dev_grow(ctx, &ctx->brid[b], oc, nc)) return DEM_ERR_HIP;
@@ -1770,7 +1770,11 @@ static int append_atoms(dem_ctx *ctx, int m, const double *x, const double *v, c
         else HIPCHK(hipMemsetAsync(ctx->rel[c] + 4 * (size_t)n0, 0, 4 * (size_t)m * sizeof(double4), s));
         HIPCHK(hipStreamSynchronize(s));
     }
-    if (ctx->have_list) launch_extend_rows(ctx->nstart[ctx->lcur], n0, m, s);
+    if (ctx->have_list) {   // through the other list's row starts, which the next rebuild writes
+        const int l = ctx->lcur;
+        launch_widen_rows(ctx->nstart[l], ctx->nstart[1 - l], n0, n1, s);
+        launch_copy_int(ctx->nstart[l], ctx->nstart[1 - l], 2 * n1 + 1, s);
+    }
     for (auto &mh : ctx->meshes) {
         if (!mh.have) continue;
         const int b = mh.cur;
@@ -2485,7 +2489,7 @@ static int capture_graph(dem_ctx *ctx)
     HIPCHK(hipStreamSynchronize(ctx->stream));   // the last rebuild may still be running
     {
         int h = 0;
-        HIPCHK(hipMemcpy(&h, ctx->nstart[ctx->lcur] + ctx->n, sizeof(int), hipMemcpyDeviceToHost));
+        HIPCHK(hipMemcpy(&h, ctx->nstart[ctx->lcur] + 2 * (size_t)ctx->n, sizeof(int), hipMemcpyDeviceToHost));
         total = h;
     }
     const int64_t want = std::max<int64_t>(2 * total, (int64_t)ctx->n * 32);
@@ -2902,10 +2906,10 @@ extern "C" int dem_get_pairs(dem_ctx *ctx, int64_t *count, int *tag_i, int *tag_
         *count = 0;
         return DEM_OK;
     }
-    std::vector<int> ns(n + 1), tg(n);
+    std::vector<int> ns(2 * (size_t)n + 1), tg(n);
     HIPCHK(hipStreamSynchronize(ctx->stream));
-    HIPCHK(hipMemcpy(ns.data(), ctx->nstart[l], (n + 1) * sizeof(int), hipMemcpyDeviceToHost));
-    const int64_t E = ns[n];
+    HIPCHK(hipMemcpy(ns.data(), ctx->nstart[l], ns.size() * sizeof(int), hipMemcpyDeviceToHost));
+    const int64_t E = ns[2 * (size_t)n];
     if (!tag_i) {
         *count = E;
         return DEM_OK;
@@ -2925,21 +2929,29 @@ extern "C" int dem_get_pairs(dem_ctx *ctx, int64_t *count, int *tag_i, int *tag_
     const int off_ref_coh = L.off_norm >= 0 ? 12 : 0;
     std::unordered_map<int64_t, int64_t> entry_of;
     if (ncoh)
-        for (int i = 0; i < n; i++)
-            for (int e = ns[i]; e < ns[i + 1]; e++)
+        for (int i = 0; i < n; i++) {
+            const Row row = list_row(ns.data(), n, i);
+            for (int q = 0; q < row.cnt; q++) {
+                const int e = row.entry(q);
                 if (((nj[e] >> 26) & 31u) == (uint32_t)kNoShift)
                     entry_of[(int64_t)i * (int64_t)n + (int64_t)(nj[e] & kJMask)] = e;
-    for (int i = 0; i < n; i++)
-        for (int e = ns[i]; e < ns[i + 1]; e++) {
+            }
+        }
+    int64_t at = -1;   // the rows of the output, one after the other
+    for (int i = 0; i < n; i++) {
+        const Row row = list_row(ns.data(), n, i);
+        for (int p = 0; p < row.cnt; p++) {
+            const int e = row.entry(p);
+            at++;
             const int j = (int)(nj[e] & kJMask);
             const int code = (int)((nj[e] >> 26) & 31u);
-            tag_i[e] = tg[i];
-            tag_j[e] = tg[j];
-            if (shift) shift[e] = code;
+            tag_i[at] = tg[i];
+            tag_j[at] = tg[j];
+            if (shift) shift[at] = code;
             const bool known = (nj[e] & (kFlagBit | kBondBit)) != 0;
-            if (flag) flag[e] = known ? 1 : 0;
+            if (flag) flag[at] = known ? 1 : 0;
             if (!hist) continue;
-            double *out = hist + (size_t)e * dnum;
+            double *out = hist + (size_t)at * dnum;
             const double *src = &hh[(size_t)e * dnum];
             // an entry without contact flags holds no contact history (zero
             // by definition); its cohesion slots are kept (zero, or what a
@@ -2960,6 +2972,7 @@ extern "C" int dem_get_pairs(dem_ctx *ctx, int64_t *count, int *tag_i, int *tag_
             }
             for (int q = off_ref_coh; q < (L.off_coh >= 0 ? L.off_coh : dnum); q++) out[k++] = known ? src[q] : 0.0;
         }
+    }
     *count = E;
     return DEM_OK;
 }
@@ -2977,15 +2990,16 @@ extern "C" int dem_set_history(dem_ctx *ctx, int64_t count, const int *tag_i, co
     std::unordered_map<int, int> idx;
     idx.reserve(n * 2 + 1);
     for (int i = 0; i < n; i++) idx[tg[i]] = i;
-    std::vector<int> cnt(n + 1, 0);
+    // every entry carries history: the rows' first parts, the second ones empty
+    std::vector<int> cnt(2 * (size_t)n + 1, 0);
     for (int64_t k = 0; k < count; k++) {
         auto it = idx.find(tag_i[k]);
         if (it == idx.end() || idx.find(tag_j[k]) == idx.end())
             return fail(ctx, DEM_ERR_ARG, "dem_set_history: unknown tag");
         cnt[it->second + 1]++;
     }
-    for (int i = 0; i < n; i++) cnt[i + 1] += cnt[i];
-    std::vector<int> fillp(cnt.begin(), cnt.end() - 1);
+    for (int i = 0; i < 2 * n; i++) cnt[i + 1] += cnt[i];
+    std::vector<int> fillp(cnt.begin(), cnt.begin() + n);
     std::vector<uint32_t> nj(std::max<int64_t>(count, 1));
     std::vector<double> hh(std::max<int64_t>(count, 1) * dnum);
     for (int64_t k = 0; k < count; k++) {
@@ -3012,7 +3026,7 @@ extern "C" int dem_set_history(dem_ctx *ctx, int64_t count, const int *tag_i, co
     }
     const int l = ctx->lcur;
     if (ensure_list_cap(ctx, l, count)) return DEM_ERR_NOMEM;
-    HIPCHK(hipMemcpy(ctx->nstart[l], cnt.data(), (n + 1) * sizeof(int), hipMemcpyHostToDevice));
+    HIPCHK(hipMemcpy(ctx->nstart[l], cnt.data(), cnt.size() * sizeof(int), hipMemcpyHostToDevice));
     if (count) {
         HIPCHK(hipMemcpy(ctx->nj[l], nj.data(), count * sizeof(uint32_t), hipMemcpyHostToDevice));
         HIPCHK(hipMemcpy(ctx->hist[l], hh.data(), count * dnum * sizeof(double), hipMemcpyHostToDevice));
@@ -3187,7 +3201,7 @@ extern "C" int dem_list_stats(dem_ctx *ctx, double *mean_neigh, double *mean_con
     if (!ctx->have_list || n == 0) return fail(ctx, DEM_ERR_ARG, "dem_list_stats: no list");
     int E = 0;
     HIPCHK(hipStreamSynchronize(ctx->stream));
-    HIPCHK(hipMemcpy(&E, ctx->nstart[ctx->lcur] + n, sizeof(int), hipMemcpyDeviceToHost));
+    HIPCHK(hipMemcpy(&E, ctx->nstart[ctx->lcur] + 2 * (size_t)n, sizeof(int), hipMemcpyDeviceToHost));
     std::vector<int> nc(n);
     HIPCHK(hipMemcpy(nc.data(), ctx->ncontact, n * sizeof(int), hipMemcpyDeviceToHost));
     double s = 0.0;
@@ -3871,7 +3885,7 @@ extern "C" int dem_autotune(dem_ctx *ctx, int reps, int *lanes, int *block, doub
     int64_t E = 0;
     {
         int h = 0;
-        HIPCHK(hipMemcpy(&h, ctx->nstart[l] + n, sizeof(int), hipMemcpyDeviceToHost));
+        HIPCHK(hipMemcpy(&h, ctx->nstart[l] + 2 * (size_t)n, sizeof(int), hipMemcpyDeviceToHost));
         E = h;
     }
     const size_t hb = sizeof(double) * (size_t)E * ctx->M.dnum, jb = sizeof(uint32_t) * (size_t)E;
@@ -3924,7 +3938,7 @@ extern "C" int dem_autotune(dem_ctx *ctx, int reps, int *lanes, int *block, doub
         return fail(ctx, DEM_ERR_HIP, "dem_autotune: copy failed");
     }
     const bool any_width = ctx->p.normal_model == 0 && ctx->p.wall_normal_model == 0 && ctx->M.cohesion == CM_OFF;
-    const int widths[] = {1, 2, 4, 8, 16, -8, -16, -32, -64};   // negative: contact-queue tiles
+    const int widths[] = {1, 2, 4, 8, 16, -8, -16, -32, -64};   // negative: tiles per wave
     const int blocks[] = {64, 128, 256};
     hipEvent_t e0, e1;
     hipEventCreate(&e0);
@@ -3945,7 +3959,8 @@ extern "C" int dem_autotune(dem_ctx *ctx, int reps, int *lanes, int *block, doub
         return r;
     };
     for (int g : widths) {
-        if (!any_width && g != 4) continue;
+        // chains with a cohesion model have one shape, other non-Hertz chains tiles
+        if (!any_width && (ctx->M.cohesion != CM_OFF ? g != 4 : g > 0)) continue;
         for (int b : blocks) {
             ctx->tune_lanes = g;
             ctx->tune_block = b;
@@ -4018,7 +4033,7 @@ extern "C" int dem_adjoint_forward(dem_ctx *ctx, int nsteps, int checkpoint_ever
     ctx->ck_ago.clear();
     {
         int h = 0;
-        HIPCHK(hipMemcpy(&h, ctx->nstart[ctx->lcur] + ctx->n, sizeof(int), hipMemcpyDeviceToHost));
+        HIPCHK(hipMemcpy(&h, ctx->nstart[ctx->lcur] + 2 * (size_t)ctx->n, sizeof(int), hipMemcpyDeviceToHost));
         ctx->adj_E = h;
     }
     if (dev_alloc(ctx, &ctx->adj_rev, (size_t)std::max<int64_t>(ctx->adj_E, 1))) return DEM_ERR_NOMEM;
@@ -4200,7 +4215,7 @@ extern "C" int dem_set_contact_shape(dem_ctx *ctx, int lanes, int block)
           || lanes == -16 || lanes == -32 || lanes == -64)
         || !(block == 0 || block == 64 || block == 128 || block == 256))
         return fail(ctx, DEM_ERR_ARG,
-                    "dem_set_contact_shape: lanes 1, 2, 4, 8, 16 (or -8, -16, -32: contact queue with tiles of that "
+                    "dem_set_contact_shape: lanes 1, 2, 4, 8, 16 (or -8, -16, -32, -64: tiles of that "
                     "many particles) and block 64, 128, 256 (0: default)");
     ctx->tune_lanes = lanes;
     ctx->tune_block = block;

@@ -18,11 +18,11 @@
 // An entry whose contact flag is still clear has never touched, so its
 // history is zero; it is neither read nor, unless it touches now, written.
 //
-// k_force_q: the same pass with a wave-level contact queue (Hertz chains,
-// the default).  Both kernels end in one per-particle epilogue (planes,
-// gravity, freeze, the force and torque written) that also integrates when
-// nothing adds to the forces after the pass, writing the new state to the
-// other state buffers.
+// k_force_t: the same pass with one list entry per lane (every chain without
+// a cohesion model, the default).  Both kernels end in one per-particle
+// epilogue (planes, gravity, freeze, the force and torque written) that also
+// integrates when nothing adds to the forces after the pass, writing the new
+// state to the other state buffers.
 //
 // k_integrate: FixNVESphere::initial_integrate / final_integrate
 // (fix_nve_sphere.cpp:134-243) with dtf = 0.5*dt, INERTIA = 0.4; mode 3 runs
@@ -106,14 +106,13 @@ __device__ inline void hist_store(double *hp, int lim, bool vec, const double (&
 // force, torque and optional per-atom outputs are written.
 template <bool MIXED, int WN>
 __device__ inline void particle_epilogue(const ForceArgs &a, int i, const double4 pi, const double4 vmi,
-                                         const double4 wi, int itype, bool fzi, const double *mat, double F[3],
-                                         double T[3], int nc)
+                                         const double4 wi, int itype, bool fzi, const double *mat, uint32_t wm,
+                                         double F[3], double T[3], int nc)
 {
     const Model &M = a.M;
     // primitive planes, in the order the fixes were defined
     double pw = 0.0;    // force of the observed plane along its axis
-    if (a.P.n) {
-        const uint32_t wm = a.wmask[i];
+    if (a.P.n && wm) {
         const double cdmw = M.cdf - 1.0;
         for (int k = 0; k < a.P.n; k++) {
             if (!(wm & (1u << k))) continue;
@@ -247,9 +246,10 @@ __global__ void __launch_bounds__(kBlock) k_force(ForceArgs a)
     c.wi[0] = wi.x; c.wi[1] = wi.y; c.wi[2] = wi.z;
     c.deltan_in = 0.0;
 
-    const int e0 = live ? a.nstart[i] : 0;
-    const int e1 = live ? a.nstart[i + 1] : 0;
-    for (int e = e0 + g; e < e1; e += G) {
+    Row row = {0, 0, 0, 0};
+    if (live) row = list_row(a.nstart, a.n, i);
+    for (int q = g; q < row.cnt; q += G) {
+        const int e = row.entry(q);
         const uint32_t w = a.nj[e];
         const int j = (int)(w & kJMask);
         const int code = (int)((w >> 26) & 31u);
@@ -328,22 +328,44 @@ __global__ void __launch_bounds__(kBlock) k_force(ForceArgs a)
     }
     if (!live || g != 0) return;
 
-    particle_epilogue<MIXED, WN>(a, i, pi, vmi, wi, itype, fzi, mat, F, T, nc);
+    particle_epilogue<MIXED, WN>(a, i, pi, vmi, wi, itype, fzi, mat, a.P.n ? a.wmask[i] : 0u, F, T, nc);
     if (a.fuse) integrate_into(a, i, pi, vmi, wi, F, T);
 }
 
 // ---------------------------------------------------------------------------
-// k_force_q: the same pass for Hertz pair and wall chains with a wave-level
-// contact queue.  A wave owns a tile of P consecutive particles, whose rows
-// form one contiguous range of the list.  The 64 lanes walk that range 64
-// entries at a time, test overlap, and append the touching entries (ballot
-// and popcount, in entry order) to a queue in LDS; every 64 queued contacts
-// are evaluated together, one per lane, so no lane idles on an entry that
-// does not touch and the partner gathers of a whole batch are in flight at
-// once.  Results go to LDS and each particle of the tile adds its own in
-// queue order, which is its list order: a sequential sum per particle,
-// deterministic, no atomics.
-constexpr int kQWaves = kBlock / 64;
+// k_force_t: a wave owns a tile of P consecutive particles.  Their entries
+// are two contiguous ranges of the list: the partners that touched at the
+// build and the others (dem_device.h).  An entry of the first range is
+// evaluated in place, one per lane: its partner's state and its history are
+// asked for together, before the overlap is known, since nearly all of them
+// still touch.  The second range is only tested, 128 entries at a time; the
+// few that touch now go to a queue in LDS and fill the lanes that the first
+// range's last batch leaves idle.  Results go to LDS, FP32 for the mixed law
+// (whose results are FP32 values) and FP64 otherwise, and every particle
+// adds its own in list order, the first range before the queue: no
+// atomics, and a sum that does not depend on where the tiles begin.
+//
+// What bounds it: the latency of its chain of gathers at 4 (mixed) or 3
+// (FP64) waves per SIMD, which the 126 / 142 registers of the law allow, with
+// 48 % of the issue slots taken by VALU.  Of the 700 B per particle of HBM
+// traffic 195 + 195 are histories; with rows of touching and other partners
+// mixed (whole rows one after the other) it was 836 B, and every entry went
+// through the test and a queue.  1M-sphere column: 276 -> 231 us mixed, 282 ->
+// 248 FP64.  Slower here: histories and state through LDS in whole lines (249
+// to 270 us), the first batch fetched ahead of the test (256, one wave per
+// SIMD fewer), tiles trimmed so that their batches fill (236).
+constexpr int kQueue = 192;   // 63 waiting and the 128 of one test
+
+template <int P, typename OutT>
+struct TileLds {
+    double4 x[P], v[P], w[P];        // the tile's state
+    OutT out[6][64];                 // a batch's forces and torques
+    int rs[2][P + 1];                // row starts, first and second range
+    int q[kQueue];                   // queued entries
+    uint8_t qo[kQueue];              // and their particles
+    uint8_t run[2][P];               // a particle's run of queued results in a batch
+    uint8_t own[16 * P];             // particle of each entry, first range then second
+};
 
 __device__ inline void wave_sync()
 {
@@ -352,224 +374,336 @@ __device__ inline void wave_sync()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-template <bool MIXED, int P>
-__global__ void __launch_bounds__(kBlock) k_force_q(ForceArgs a)
+// One entry's DN history slots, in the widest pieces their alignment allows
+template <int DN, int HN>
+__device__ inline void slots_load(const double *hp, double (&h)[HN])
 {
-    static_assert(P <= 64, "a tile fits one wave");
-    __shared__ int s_rs[kQWaves][P + 1];
-    __shared__ double4 s_x[kQWaves][P];
-    __shared__ double4 s_v[kQWaves][P], s_w[kQWaves][P];   // the tile's velocity/mass, spin/meta
-    __shared__ int s_q[kQWaves][128], s_qo[kQWaves][128];
-    __shared__ uint32_t s_qw[kQWaves][128];          // list word of the queued entry
-    __shared__ double s_qd[kQWaves][4][128];         // its separation x_i - x_j, partner radius
-    // per-contact results; the mixed law's are FP32 values, kept exactly
-    using OutT = typename std::conditional<MIXED, float, double>::type;
-    __shared__ OutT s_out[kQWaves][6][64];
-    __shared__ int s_run0[kQWaves][P], s_run1[kQWaves][P];
+    static_assert(HN >= DN, "room for the slots");
+    if constexpr (DN % 2 == 0) {
+#pragma unroll
+        for (int q = 0; q < DN / 2; q++) {
+            const double2 v = reinterpret_cast<const double2 *>(hp)[q];
+            h[2 * q] = v.x;
+            h[2 * q + 1] = v.y;
+        }
+    } else {
+#pragma unroll
+        for (int q = 0; q < DN; q++) h[q] = hp[q];
+    }
+}
 
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+template <int DN, int HN>
+__device__ inline void slots_store(double *hp, const double (&h)[HN])
+{
+    if constexpr (DN % 2 == 0) {
+#pragma unroll
+        for (int q = 0; q < DN / 2; q++) reinterpret_cast<double2 *>(hp)[q] = make_double2(h[2 * q], h[2 * q + 1]);
+    } else {
+#pragma unroll
+        for (int q = 0; q < DN; q++) hp[q] = h[q];
+    }
+}
+
+// contact_close with the chain's layout known; true if the flag stays set
+template <int NM, int DN>
+__device__ inline bool slots_close(double *hp)
+{
+    constexpr int s0 = chain_off_shear(NM);
+    if constexpr (NM != NM_HERTZ)
+#pragma unroll
+        for (int q = 0; q < 10; q++) hp[q] = 0.0;
+#pragma unroll
+    for (int q = s0; q < DN; q++) hp[q] = 0.0;
+    return NM == NM_HERTZ;
+}
+
+// DN: history slots of the pair chain (its rolling history included or not)
+template <bool MIXED, int NM, int WN, int DN, int P>
+__global__ void __launch_bounds__(kBlock) k_force_t(ForceArgs a)
+{
+    static_assert(P == 8 || P == 16 || P == 32 || P == 64, "a tile fits one wave");
+    static_assert(!MIXED || NM == NM_HERTZ, "the mixed law is Hertz's");
+    using OutT = typename std::conditional<MIXED, float, double>::type;
+    using Lds = TileLds<P, OutT>;
+    extern __shared__ __align__(16) char s_raw[];
+    // lanes that sum: P particles times kParts groups of kPer components
+    constexpr int kParts = P == 8 ? 6 : (P == 16 ? 3 : (P == 32 ? 2 : 1));
+    constexpr int kPer = 6 / kParts;
+    constexpr int kOwn = 16 * P;
+    constexpr int RH = DN > chain_off_shear(NM) + 3 ? 1 : 0;
+    static_assert(DN == chain_off_shear(NM) + 3 + 3 * RH, "shear, then rolling");
+    // the mixed law asks the model whether it rolls, so its slots always exist
+    constexpr int HN = MIXED ? chain_max_dnum(NM) : DN;
+
+    // the wave's number in the block is the same for its lanes: every address
+    // of the tile stays in scalar registers
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int blk = xcd_block(blockIdx.x, gridDim.x);
     const int p0 = (blk * (int)(blockDim.x >> 6) + wv) * P;
     if (p0 >= a.n) return;   // uniform over the wave
     if (a.halt && *a.halt) return;
+    Lds &L = reinterpret_cast<Lds *>(s_raw)[wv];
     const int np = min(P, a.n - p0);
     const Model &M = a.M;
-    const int dnum = M.dnum;
+    uint32_t wm = 0;
     if (lane < np) {
-        s_x[wv][lane] = a.xr[p0 + lane];
-        s_v[wv][lane] = a.vm[p0 + lane];
-        s_w[wv][lane] = a.wt[p0 + lane];
+        L.x[lane] = a.xr[p0 + lane];
+        L.v[lane] = a.vm[p0 + lane];
+        L.w[lane] = a.wt[p0 + lane];
+        if (a.P.n) wm = a.wmask[p0 + lane];
+        L.rs[0][lane] = a.nstart[p0 + lane];
+        L.rs[1][lane] = a.nstart[a.n + p0 + lane];
     }
-    // row starts of the tile and, from lane 0, the end of its last row (a
-    // tile of 64 has no 65th lane)
-    if (lane < np) s_rs[wv][lane] = a.nstart[p0 + lane];
-    if (lane == 0) s_rs[wv][np] = a.nstart[p0 + np];
+    const int A0 = a.nstart[p0], nA = a.nstart[p0 + np] - A0;
+    const int B0 = a.nstart[a.n + p0], nB = a.nstart[a.n + p0 + np] - B0;
+    if (lane == 0) {   // the ends of the last rows
+        L.rs[0][np] = A0 + nA;
+        L.rs[1][np] = B0 + nB;
+    }
     wave_sync();
-    const int E0 = s_rs[wv][0], E1 = s_rs[wv][np];
-    const double cdm = M.cdf * M.cdf;
-    double F[3] = {0.0, 0.0, 0.0}, T[3] = {0.0, 0.0, 0.0};
-    int nc = 0;
-    int qlen = 0;
-
-    // evaluate queue items [0, m): one contact per lane, then each owner adds
-    // its run of results
-    auto eval_batch = [&](int m) {
-        if (lane < np) {
-            s_run0[wv][lane] = 0;
-            s_run1[wv][lane] = 0;
+    // particle of each entry, written row by row; past kOwn entries by search
+    if (lane < np) {
+        for (int t = L.rs[0][lane] - A0; t < min(L.rs[0][lane + 1] - A0, kOwn); t++) L.own[t] = (uint8_t)lane;
+        for (int t = L.rs[1][lane] - B0 + nA; t < min(L.rs[1][lane + 1] - B0 + nA, kOwn); t++)
+            L.own[t] = (uint8_t)lane;
+    }
+    wave_sync();
+    auto owner = [&](int range, int t) {   // t: entry of the tile, first range then second
+        if (t < kOwn) return (int)L.own[t];
+        const int e = range ? B0 + (t - nA) : A0 + t;
+        int lo = 0, hi = np - 1;   // the last row starting at or before e
+        while (lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if (L.rs[range][mid] <= e) lo = mid;
+            else hi = mid - 1;
         }
-        wave_sync();
-        double dF[3] = {0.0, 0.0, 0.0}, dT[3] = {0.0, 0.0, 0.0};
-        if (lane < m) {
-            const int e = s_q[wv][lane];
-            const int k = s_qo[wv][lane];
-            const uint32_t w = s_qw[wv][lane];
-            const int j = (int)(w & kJMask);
-            // the partner's velocity, spin and the entry's history are
-            // independent loads, all in flight together
-            double4 vmj, wj;
+        return lo;
+    };
+    const double cdm = M.cdf * M.cdf;
+    double acc[kPer];
+#pragma unroll
+    for (int c = 0; c < kPer; c++) acc[c] = 0.0;
+    int nc = 0;
+
+    // evaluate one batch: m1 entries of the first range from its entry t0 on,
+    // then mq of the queue's first entries
+    auto batch = [&](int t0, int m1, int mq) {
+        const bool act = lane < m1 + mq;
+        bool touch = false;
+        int k = 0;
+#pragma unroll
+        for (int c = 0; c < 6; c++) L.out[c][lane] = (OutT)0;
+        int e = A0 + t0 + lane;
+        if (act) {
+            if (lane >= m1) e = L.q[lane - m1];
+            k = lane < m1 ? owner(0, t0 + lane) : (int)L.qo[lane - m1];
+            // the partner's state and the history are asked for together, before
+            // the overlap is known
+            const uint32_t bw = a.nj[e];
+            double *hp = a.hist + (size_t)e * DN;
+            double bh[HN];
+            slots_load<DN>(hp, bh);   // allocated, whatever it holds
+            const int j = (int)(bw & kJMask);
+            const double4 bx = a.xr[j];
+            double4 bv, bs;
             if (MIXED && a.rec) {
                 const float4 r0 = a.rec[2 * (size_t)j], r1 = a.rec[2 * (size_t)j + 1];
-                vmj = make_double4(r0.x, r0.y, r0.z, r0.w);
-                wj = make_double4(r1.x, r1.y, r1.z, (double)__float_as_int(r1.w));
+                bv = make_double4(r0.x, r0.y, r0.z, r0.w);
+                bs = make_double4(r1.x, r1.y, r1.z, (double)__float_as_int(r1.w));
             } else {
-                vmj = a.vm[j];
-                wj = a.wt[j];
+                bv = a.vm[j];
+                bs = a.wt[j];
             }
-            const double radj = s_qd[wv][3][lane];
-            const double4 pi = s_x[wv][k], vmi = s_v[wv][k], wi = s_w[wv][k];
-            const int metai = (int)wi.w;
-            const double *mat = a.mat + (size_t)meta_inst(metai) * kMatStride;
+            const double4 pi = L.x[k];
+            const int code = (int)((bw >> 26) & 31u);
+            double xj0 = bx.x, xj1 = bx.y, xj2 = bx.z;
+            if (code != kNoShift) {
+                const double3 im = image_of(bx, code, M.prd);
+                xj0 = im.x; xj1 = im.y; xj2 = im.z;
+            }
             ContactIn c;
-            c.is_wall = false;
-            c.itype = meta_type(metai);
-            c.radi = pi.w;
-            c.mi = vmi.w;
-            c.vi[0] = vmi.x; c.vi[1] = vmi.y; c.vi[2] = vmi.z;
-            c.wi[0] = wi.x; c.wi[1] = wi.y; c.wi[2] = wi.z;
-            c.deltan_in = 0.0;
-            c.delta[0] = s_qd[wv][0][lane];
-            c.delta[1] = s_qd[wv][1][lane];
-            c.delta[2] = s_qd[wv][2][lane];
+            c.delta[0] = pi.x - xj0;
+            c.delta[1] = pi.y - xj1;
+            c.delta[2] = pi.z - xj2;
             const double rsq = c.delta[0] * c.delta[0] + c.delta[1] * c.delta[1] + c.delta[2] * c.delta[2];
-            const double r = sqrt(rsq);
-            if (r < 1e-20) atomicOr(a.err, 1);
-            const int metaj = (int)wj.w;
-            c.jtype = meta_type(metaj);
-            c.radj = radj;
-            c.mj = vmj.w;
-            double meff = c.mi * c.mj / (c.mi + c.mj);
-            if (M.freeze_on && meta_frozen(metai)) meff = c.mj;
-            if (M.freeze_on && meta_frozen(metaj)) meff = c.mi;
-            c.meff = meff;
-            c.r = r;
-            c.rinv = 1.0 / r;
-            c.radsum = pi.w + radj;
-            c.vj[0] = vmj.x; c.vj[1] = vmj.y; c.vj[2] = vmj.z;
-            c.wj[0] = wj.x; c.wj[1] = wj.y; c.wj[2] = wj.z;
-            constexpr int HN = chain_max_dnum(NM_HERTZ);
-            double h[HN];
-            double *hp = a.hist + (size_t)e * dnum;
-            const bool known = (w & kFlagBit) != 0;
-            const bool vec = (dnum & 1) == 0;
-            hist_load(hp, dnum, vec, known, h);
-            if (MIXED) contact_mixed(M, mat, c, h, a.shearupdate, dF, dT);
-            else contact_fp64<NM_HERTZ>(M, M.lp, mat, c, h, a.shearupdate, dF, dT);
-            if (a.shearupdate || !known) hist_store(hp, dnum, vec, h);
-            if (!known) a.nj[e] = w | kFlagBit;
-            if (lane == 0 || s_qo[wv][lane - 1] != k) s_run0[wv][k] = lane;
-            if (lane == m - 1 || s_qo[wv][lane + 1] != k) s_run1[wv][k] = lane + 1;
+            c.radsum = pi.w + bx.w;
+            touch = rsq < c.radsum * c.radsum;
+            if (touch) {
+                const double4 vmi = L.v[k], wi = L.w[k];
+                const int metai = (int)wi.w, metaj = (int)bs.w;
+                const double *mat = a.mat + (size_t)meta_inst(metai) * kMatStride;
+                c.is_wall = false;
+                c.itype = meta_type(metai);
+                c.jtype = meta_type(metaj);
+                c.radi = pi.w;
+                c.radj = bx.w;
+                c.mi = vmi.w;
+                c.mj = bv.w;
+                c.vi[0] = vmi.x; c.vi[1] = vmi.y; c.vi[2] = vmi.z;
+                c.wi[0] = wi.x; c.wi[1] = wi.y; c.wi[2] = wi.z;
+                c.vj[0] = bv.x; c.vj[1] = bv.y; c.vj[2] = bv.z;
+                c.wj[0] = bs.x; c.wj[1] = bs.y; c.wj[2] = bs.z;
+                c.deltan_in = 0.0;
+                const double r = sqrt(rsq);
+                if (r < 1e-20) atomicOr(a.err, 1);
+                double meff = c.mi * c.mj / (c.mi + c.mj);
+                if (M.freeze_on && meta_frozen(metai)) meff = c.mj;
+                if (M.freeze_on && meta_frozen(metaj)) meff = c.mi;
+                c.meff = meff;
+                c.r = r;
+                c.rinv = 1.0 / r;
+                // an unflagged entry has no history yet
+                const bool known = (bw & kFlagBit) != 0;
+                if (!known)
+#pragma unroll
+                    for (int q = 0; q < HN; q++) bh[q] = 0.0;
+                double dF[3], dT[3];
+                if constexpr (MIXED)
+                    contact_mixed(M, mat, c, bh, a.shearupdate, dF, dT);
+                else
+                    contact_fp64<NM, false, RH>(M, M.lp, mat, c, bh, a.shearupdate, dF, dT);
+                // the hysteretic models write their state even in set-up passes
+                if (a.shearupdate || !known || NM != NM_HERTZ) slots_store<DN>(hp, bh);
+                if (!known) a.nj[e] = bw | kFlagBit;
+#pragma unroll
+                for (int q = 0; q < 3; q++) {
+                    L.out[q][lane] = (OutT)dF[q];
+                    L.out[3 + q][lane] = (OutT)dT[q];
+                }
+            } else if (rsq < cdm * c.radsum * c.radsum) {
+                // surfacesClose: history reset; a hysteretic chain also clears
+                // its contact flag, so the entry no longer carries at a rebuild
+                if (!slots_close<NM, DN>(hp)) a.nj[e] = bw & ~kFlagBit;
+            }
         }
-        s_out[wv][0][lane] = (OutT)dF[0]; s_out[wv][1][lane] = (OutT)dF[1]; s_out[wv][2][lane] = (OutT)dF[2];
-        s_out[wv][3][lane] = (OutT)dT[0]; s_out[wv][4][lane] = (OutT)dT[1]; s_out[wv][5][lane] = (OutT)dT[2];
+        const uint64_t tm = __ballot(touch);
+        if (tm == 0) return;
+        if (mq) {
+            if (lane < P) L.run[0][lane] = L.run[1][lane] = 0;
+            wave_sync();
+            if (act && lane >= m1) {
+                if (lane == m1 || L.qo[lane - m1 - 1] != k) L.run[0][k] = (uint8_t)lane;
+                if (lane == m1 + mq - 1 || L.qo[lane - m1 + 1] != k) L.run[1][k] = (uint8_t)(lane + 1);
+            }
+        }
         wave_sync();
-        if (lane < np) {
-            const int l1 = s_run1[wv][lane];
-            for (int l = s_run0[wv][lane]; l < l1; l++) {
-                F[0] += (double)s_out[wv][0][l]; F[1] += (double)s_out[wv][1][l]; F[2] += (double)s_out[wv][2][l];
-                T[0] += (double)s_out[wv][3][l]; T[1] += (double)s_out[wv][4][l]; T[2] += (double)s_out[wv][5][l];
-                nc++;
+        const int pl = lane & (P - 1), part = lane / P;
+        const bool sums = pl < np && part < kParts;
+        if (sums) {
+            const int l0 = max(L.rs[0][pl] - A0 - t0, 0), l1 = min(L.rs[0][pl + 1] - A0 - t0, m1);
+            for (int l = l0; l < l1; l++)
+#pragma unroll
+                for (int c = 0; c < kPer; c++) acc[c] += (double)L.out[part * kPer + c][l];
+            if (a.ncontact && l1 > l0) nc += __popcll((tm >> l0) & (l1 - l0 == 64 ? ~0ull : (1ull << (l1 - l0)) - 1ull));
+            if (mq) {
+                const int q1 = L.run[1][pl];
+                for (int l = L.run[0][pl]; l < q1; l++) {
+#pragma unroll
+                    for (int c = 0; c < kPer; c++) acc[c] += (double)L.out[part * kPer + c][l];
+                    nc++;
+                }
             }
         }
         wave_sync();
     };
 
-    // software pipeline: the next 64 entries' list words and partner
-    // positions are in flight while this group is tested and queued (and
-    // while a batch of contacts is evaluated)
-    uint32_t w_next = 0;
-    double4 pj_next = make_double4(0.0, 0.0, 0.0, 0.0);
-    if (E0 + lane < E1) {
-        w_next = a.nj[E0 + lane];
-        pj_next = a.xr[w_next & kJMask];
-    }
-    for (int base = E0; base < E1; base += 64) {
-        const int e = base + lane;
-        bool touch = false;
-        int owner = 0;
-        uint32_t w = w_next;
-        const double4 pj = pj_next;
-        if (e + 64 < E1) {
-            w_next = a.nj[e + 64];
-            pj_next = a.xr[w_next & kJMask];
+    // test the second range's entries [base, base + 128), touching ones to the queue
+    int qlen = 0;
+    auto filter = [&](int base) {
+        uint32_t w[2];
+        double4 pj[2];
+        bool in[2];
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            in[u] = base + 64 * u + lane < nB;
+            w[u] = in[u] ? a.nj[B0 + base + 64 * u + lane] : 0u;
         }
-        double dx = 0.0, dy = 0.0, dz = 0.0, rj = 0.0;
-        if (e < E1) {
-            int lo = 0, hi = np - 1;   // owner: the last row starting at or before e
-            while (lo < hi) {
-                const int mid = (lo + hi + 1) >> 1;
-                if (s_rs[wv][mid] <= e) lo = mid;
-                else hi = mid - 1;
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+            if (in[u]) pj[u] = a.xr[w[u] & kJMask];
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            if (base + 64 * u >= nB) break;
+            const int t = base + 64 * u + lane;
+            bool touch = false;
+            int k = 0;
+            if (in[u]) {
+                k = owner(1, nA + t);
+                const double4 pi = L.x[k];
+                const int code = (int)((w[u] >> 26) & 31u);
+                double xj0 = pj[u].x, xj1 = pj[u].y, xj2 = pj[u].z;
+                if (code != kNoShift) {
+                    const double3 im = image_of(pj[u], code, M.prd);
+                    xj0 = im.x; xj1 = im.y; xj2 = im.z;
+                }
+                const double dx = pi.x - xj0, dy = pi.y - xj1, dz = pi.z - xj2;
+                const double rsq = dx * dx + dy * dy + dz * dz;
+                const double radsum = pi.w + pj[u].w;
+                touch = rsq < radsum * radsum;
+                if (!touch && rsq < cdm * radsum * radsum) {   // as in the batch
+                    const int e = B0 + t;
+                    if (!slots_close<NM, DN>(a.hist + (size_t)e * DN)) a.nj[e] = w[u] & ~kFlagBit;
+                }
             }
-            owner = lo;
-            const int code = (int)((w >> 26) & 31u);
-            const double4 pi = s_x[wv][owner];
-            double xj0 = pj.x, xj1 = pj.y, xj2 = pj.z;
-            if (code != kNoShift) {
-                const double3 im = image_of(pj, code, M.prd);
-                xj0 = im.x; xj1 = im.y; xj2 = im.z;
+            const uint64_t bm = __ballot(touch);
+            if (touch) {
+                const int pos = qlen + __popcll(bm & ((1ull << lane) - 1ull));
+                L.q[pos] = B0 + t;
+                L.qo[pos] = (uint8_t)k;
             }
-            dx = pi.x - xj0;
-            dy = pi.y - xj1;
-            dz = pi.z - xj2;
-            const double rsq = dx * dx + dy * dy + dz * dz;
-            rj = pj.w;
-            const double radsum = pi.w + pj.w;
-            touch = rsq < radsum * radsum;
-            if (!touch && rsq < cdm * radsum * radsum) {
-                // surfacesClose: history reset (Hertz keeps its contact flag)
-                contact_close(M.lp, a.hist + (size_t)e * dnum);
-            }
-        }
-        const uint64_t bm = __ballot(touch);
-        if (touch) {
-            const int pos = qlen + __popcll(bm & ((1ull << lane) - 1ull));
-            s_q[wv][pos] = e;
-            s_qo[wv][pos] = owner;
-            s_qw[wv][pos] = w;
-            s_qd[wv][0][pos] = dx;
-            s_qd[wv][1][pos] = dy;
-            s_qd[wv][2][pos] = dz;
-            s_qd[wv][3][pos] = rj;
-        }
-        qlen += __popcll(bm);
-        wave_sync();
-        if (qlen >= 64) {
-            eval_batch(64);
-            const int rest = qlen - 64;
-            int tq = 0, to = 0;
-            uint32_t tw = 0;
-            double t0 = 0.0, t1 = 0.0, t2 = 0.0, t3 = 0.0;
-            if (lane < rest) {
-                tq = s_q[wv][64 + lane];
-                to = s_qo[wv][64 + lane];
-                tw = s_qw[wv][64 + lane];
-                t0 = s_qd[wv][0][64 + lane];
-                t1 = s_qd[wv][1][64 + lane];
-                t2 = s_qd[wv][2][64 + lane];
-                t3 = s_qd[wv][3][64 + lane];
-            }
+            qlen += __popcll(bm);
             wave_sync();
-            if (lane < rest) {
-                s_q[wv][lane] = tq;
-                s_qo[wv][lane] = to;
-                s_qw[wv][lane] = tw;
-                s_qd[wv][0][lane] = t0;
-                s_qd[wv][1][lane] = t1;
-                s_qd[wv][2][lane] = t2;
-                s_qd[wv][3][lane] = t3;
-            }
+        }
+    };
+    // Test the second range while the queue has room, evaluate the first
+    // range, with the queue's first entries in its last batch's idle lanes,
+    // then what is left of the queue and of the second range: every
+    // particle's results come in list order.
+    for (int b = 0, t0 = 0;;) {
+        if (b < nB && qlen < 64 && (t0 == 0 || t0 == nA)) {
+            filter(b);
+            b += 128;
+            continue;
+        }
+        const int m1 = min(64, nA - t0);
+        const int mq = t0 + m1 == nA ? min(qlen, 64 - m1) : 0;
+        if (m1 + mq == 0) break;
+        batch(t0, m1, mq);
+        t0 += m1;
+        qlen -= mq;
+        if (mq && qlen) {   // the rest to the front
+            int tq[3];
+            uint8_t to[3];
+#pragma unroll
+            for (int u = 0; u < 3; u++)
+                if (64 * u + lane < qlen) {
+                    tq[u] = L.q[mq + 64 * u + lane];
+                    to[u] = L.qo[mq + 64 * u + lane];
+                }
             wave_sync();
-            qlen = rest;
+#pragma unroll
+            for (int u = 0; u < 3; u++)
+                if (64 * u + lane < qlen) {
+                    L.q[64 * u + lane] = tq[u];
+                    L.qo[64 * u + lane] = to[u];
+                }
+            wave_sync();
         }
     }
-    if (qlen > 0) eval_batch(qlen);
+
+    // a particle's components back to its own lane
+    double F[3], T[3];
+#pragma unroll
+    for (int c = 0; c < 6; c++) {
+        const double v = kParts == 1 ? acc[c % kPer] : __shfl(acc[c % kPer], (c / kPer) * P + (lane & (P - 1)), 64);
+        (c < 3 ? F[c] : T[c - 3]) = v;
+    }
     if (lane < np) {
         const int i = p0 + lane;
-        const double4 pi = s_x[wv][lane], vmi = s_v[wv][lane], wi = s_w[wv][lane];
+        const double4 pi = L.x[lane], vmi = L.v[lane], wi = L.w[lane];
         const int metai = (int)wi.w;
         const double *mat = a.mat + (size_t)meta_inst(metai) * kMatStride;
-        particle_epilogue<MIXED, NM_HERTZ>(a, i, pi, vmi, wi, meta_type(metai), meta_frozen(metai), mat, F, T, nc);
+        particle_epilogue<MIXED, WN>(a, i, pi, vmi, wi, meta_type(metai), meta_frozen(metai), mat, wm, F, T, nc);
         if (a.fuse) integrate_into(a, i, pi, vmi, wi, F, T);
     }
 }
@@ -581,58 +715,76 @@ static int padded_blocks(long long threads, int block = kBlock)
 }
 
 // Shape of the pass: ForceArgs::lanes/block (set by the autotuner or by
-// hand), else DEM_CONTACT_LANES, else the default.  lanes > 0: lane groups
-// of that width per particle (k_force); lanes < 0: contact queue with tiles
-// of -lanes particles per wave (k_force_q, Hertz chains).  Default: queue
-// tiles of 32 with 256-thread blocks, the fastest measured on MI355X for
-// the 1M-sphere column (0.33 ms per pass against 0.41 ms for 4-lane groups,
-// FP64 0.33 against 0.44).
-static int contact_shape(const ForceArgs &a)
+// hand), else DEM_CONTACT_LANES, else by the particle count.  lanes > 0: lane
+// groups of that width per particle (k_force, Hertz chains); lanes < 0: tiles
+// of -lanes particles per wave (k_force_t).
+//
+// By the count: a small tile is the shorter chain of batches, a large one
+// has fewer half-empty batches and less per-wave work.  The smallest that
+// keeps the waves to what the chip holds at once (256 CUs, 3-4 per SIMD) is
+// the fastest up to there: column of n spheres, mixed, us per pass with tiles
+// of 8 / 16 / 32: 20,000 13.5 / 15.5 / 17.8; 50,000 22.0 / 20.0 / 20.8;
+// 200,000 62 / 51 / 46.  From there on 32, and for FP64, whose pass runs at 3
+// waves per SIMD whatever the tile, 64 once both keep every slot busy for many
+// rounds (200,000 55 / 59 with 32 / 64; 500,000 114 / 110; 1M 262 / 248; mixed
+// 231 / 241).
+static int contact_shape(const ForceArgs &a, bool mixed)
 {
     if (a.lanes) return a.lanes;
-    static int g = 0;
-    if (g == 0) {
+    static const int env = [] {
         const char *s = getenv("DEM_CONTACT_LANES");
-        g = s ? atoi(s) : -32;
-        if (g != 1 && g != 2 && g != 4 && g != 8 && g != 16 && g != -8 && g != -16 && g != -32 && g != -64) g = -32;
-    }
-    return g;
+        const int g = s ? atoi(s) : 0;
+        for (int v : {1, 2, 4, 8, 16, -8, -16, -32, -64})
+            if (g == v) return g;
+        return 0;
+    }();
+    if (env) return env;
+    constexpr int kWaves = 3584;
+    if (a.n <= 8 * kWaves) return -8;
+    if (a.n <= 16 * kWaves) return -16;
+    return !mixed && a.n > 112 * kWaves ? -64 : -32;
 }
 
 bool force_can_fuse(const ForceArgs &a) { return a.M.cohesion == CM_OFF; }
 
-// Hertz pairs with Hertz walls (the common case) take any group width;
-// other model combinations run with 4 lanes per particle.
+template <bool MIXED, int NM, int WN, int P>
+static void launch_tile(const ForceArgs &a, int B, hipStream_t s)
+{
+    using OutT = typename std::conditional<MIXED, float, double>::type;
+    constexpr int D0 = chain_off_shear(NM) + 3;
+    const int nb = padded_blocks(((long long)a.n + P - 1) / P * 64, B);
+    const size_t lds = (B / 64) * sizeof(TileLds<P, OutT>);
+    if (a.M.dnum == D0) k_force_t<MIXED, NM, WN, D0, P><<<nb, B, lds, s>>>(a);
+    else k_force_t<MIXED, NM, WN, D0 + 3, P><<<nb, B, lds, s>>>(a);
+}
+
+// Hertz pairs with Hertz walls (the common case) take any shape; other model
+// combinations run in tiles.
 template <bool MIXED, int NM, int WN>
 static void launch_nm(const ForceArgs &a, hipStream_t s)
 {
-    const int B = a.block ? a.block : kBlock;
-    const int shape = contact_shape(a);
+    const int shape = contact_shape(a, MIXED);
+    // a tile's wave shares nothing with the others of its block
+    const int B = a.block ? a.block : (shape > 0 ? kBlock : 64);
     if constexpr (NM == NM_HERTZ && WN == NM_HERTZ) {
-        if (shape < 0) {
-            const int P = -shape;
-            const long long tiles = ((long long)a.n + P - 1) / P;
-            const int nb = padded_blocks(tiles * 64, B);
-            switch (P) {
-            case 8: k_force_q<MIXED, 8><<<nb, B, 0, s>>>(a); return;
-            case 32: k_force_q<MIXED, 32><<<nb, B, 0, s>>>(a); return;
-            case 64: k_force_q<MIXED, 64><<<nb, B, 0, s>>>(a); return;
-            default: k_force_q<MIXED, 16><<<nb, B, 0, s>>>(a); return;
-            }
-        }
-    }
-    const int G = (NM == NM_HERTZ && WN == NM_HERTZ && shape > 0) ? shape : 4;
-    const int nb = padded_blocks((long long)a.n * G, B);
-    if constexpr (NM == NM_HERTZ && WN == NM_HERTZ) {
-        switch (G) {
+        const int nb = padded_blocks((long long)a.n * (shape > 0 ? shape : 1), B);
+        switch (shape) {
         case 1: k_force<MIXED, 1, NM, WN><<<nb, B, 0, s>>>(a); return;
         case 2: k_force<MIXED, 2, NM, WN><<<nb, B, 0, s>>>(a); return;
+        case 4: k_force<MIXED, 4, NM, WN><<<nb, B, 0, s>>>(a); return;
         case 8: k_force<MIXED, 8, NM, WN><<<nb, B, 0, s>>>(a); return;
         case 16: k_force<MIXED, 16, NM, WN><<<nb, B, 0, s>>>(a); return;
         default: break;
         }
     }
-    k_force<MIXED, 4, NM, WN><<<nb, B, 0, s>>>(a);
+    if constexpr (WN == NM_HERTZ)
+        switch (shape) {
+        case -8: launch_tile<MIXED, NM, WN, 8>(a, B, s); return;
+        case -16: launch_tile<MIXED, NM, WN, 16>(a, B, s); return;
+        case -64: launch_tile<MIXED, NM, WN, 64>(a, B, s); return;
+        default: break;
+        }
+    launch_tile<MIXED, NM, WN, 32>(a, B, s);
 }
 
 // with a cohesion model: FP64, 4 lanes per particle

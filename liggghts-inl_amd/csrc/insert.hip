@@ -17,7 +17,8 @@
 // k_region_sums  count, volume and mass of the particles inside a block
 //                (FixInsertPack::calc_ninsert_this), fixed-order partials
 // k_tmpl_inside  inside tests of a multisphere template's Monte Carlo points
-// k_extend_rows  empty previous-list rows for appended atoms
+// k_widen_rows   empty previous-list rows for appended atoms
+// k_extend_rows  the same for mesh candidate rows
 // k_stream_release  fix insert/stream's end_of_step: atoms awaiting release
 //                ride the extrusion at the normal velocity
 #include "kernels.h"
@@ -315,6 +316,19 @@ __global__ void __launch_bounds__(kBlock) k_extend_rows(int *start, int from, in
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= count) return;
     start[from + 1 + t] = start[from];
+}
+
+// row starts re-laid for more particles: the touching parts, then the others
+__global__ void __launch_bounds__(kBlock) k_widen_rows(const int *src, int *dst, int n0, int n1)
+{
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t > 2 * n1) return;
+    dst[t] = src[t <= n1 ? min(t, n0) : n0 + min(t - n1, n0)];
+}
+
+void launch_widen_rows(const int *src, int *dst, int n0, int n1, hipStream_t s)
+{
+    k_widen_rows<<<(2 * n1 + 1 + kBlock - 1) / kBlock, kBlock, 0, s>>>(src, dst, n0, n1);
 }
 
 void launch_extend_rows(int *start, int from, int count, hipStream_t s)

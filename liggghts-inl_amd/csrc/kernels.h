@@ -112,9 +112,9 @@ struct NeighArgs {
     const double4 *wt;   // new order (instance in meta)
     const int *tag;      // new order
     const int *cstart;   // per key, exclusive prefix + total at nkeys
-    int *count;          // per atom (count pass)
+    int *count;          // per atom: touching partners, then (at n + i) the others (count pass)
     int *maxcount;
-    const int *nstart;   // per atom (fill pass)
+    const int *nstart;   // 2n + 1, scanned counts (fill pass)
     uint32_t *nj;
     double *hist;
     // previous list, old index space
@@ -297,8 +297,9 @@ void launch_scatter(const uint32_t *key, int *cursor, int *sorted, int n, hipStr
 void launch_cellsort(const int *cstart, int *sorted, int nkeys, hipStream_t s);
 void launch_permute(const PermuteArgs &a, hipStream_t s);
 void launch_neigh_count(const NeighArgs &a, hipStream_t s);
-// *maxcount = max(*maxcount, max of count[0..n))
-void launch_row_max(const int *count, int n, int *maxcount, hipStream_t s);
+// *maxcount = max(*maxcount, max of count[i]), with two parts of
+// count[i] + count[n + i], over i < n
+void launch_row_max(const int *count, int n, int parts, int *maxcount, hipStream_t s);
 void launch_neigh_fill(const NeighArgs &a, hipStream_t s);
 
 // fix setforce / fix aveforce on a group (FixSetForce::post_force,
@@ -423,6 +424,9 @@ void launch_region_sums(const double4 *xr, const double4 *vm, int n, const doubl
 // inside[k] = 1 when point k lies inside one of the nsph spheres (xs, rs)
 void launch_tmpl_inside(const double *pts, int npts, const double *xs, const double *rs, int nsph, uint8_t *inside,
                         hipStream_t s);
+// row starts of a list of n0 particles for n1 >= n0, the new rows empty:
+// src 2 n0 + 1 entries, dst 2 n1 + 1
+void launch_widen_rows(const int *src, int *dst, int n0, int n1, hipStream_t s);
 // start[from + 1 .. from + count] = start[from]
 void launch_extend_rows(int *start, int from, int count, hipStream_t s);
 

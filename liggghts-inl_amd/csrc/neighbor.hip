@@ -449,33 +449,33 @@ __global__ void __launch_bounds__(kBlock) k_neigh(NeighArgs a)
     // the particle's previous row into LDS: partner tag of every flagged
     // entry (0 = cannot match; tags are positive), its first kOld entries
     // (a longer row is searched in memory past them)
-    int ob = 0, oe = 0;
+    Row orow = {0, 0, 0, 0};
     if (OLD && a.have_old) {
         const int o = a.perm[p];
-        ob = a.onstart[o];
-        oe = a.onstart[o + 1];
-        for (int k = lane; k < min(oe - ob, kOld); k += W) {
-            const uint32_t ow = a.onj[ob + k];
+        orow = list_row(a.onstart, a.n, o);
+        for (int k = lane; k < min(orow.cnt, kOld); k += W) {
+            const uint32_t ow = a.onj[orow.entry(k)];
             s_ot[wv][k] = (ow & (kFlagBit | kBondBit)) ? a.otag[ow & kJMask] : 0;
         }
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
-    const int onl = min(oe - ob, kOld);
-    const int ebase = FILL ? a.nstart[p] : 0;
+    const int onl = min(orow.cnt, kOld);
     // a list longer than the allocation (possible only when the rebuild runs
     // inside a captured graph, sized beforehand) is reported, not written
-    if (FILL && (int64_t)a.nstart[a.n] > a.ecap) {
+    if (FILL && (int64_t)a.nstart[2 * a.n] > a.ecap) {
         if (lane == 0) atomicOr(a.err, 8);
         return;
     }
-    int written = 0;
+    int written = 0, wtouch = 0;
     // the fill pass writes a row in two sweeps, touching entries then the
     // others (each in scan order): the order the staged rows are compacted
     // in, so both paths give the same list
     constexpr int kSweeps = FILL ? 2 : 1;
-    for (int sweep = 0; sweep < kSweeps; sweep++)
+    for (int sweep = 0; sweep < kSweeps; sweep++) {
+    const int ebase = FILL ? a.nstart[sweep ? a.n + p : p] : 0;
+    if (FILL) written = 0;
     for (int c0 = 0; c0 < total; c0 += W) {
         const int c = c0 + lane;
         bool pass = false, touch = false;
@@ -528,26 +528,27 @@ __global__ void __launch_bounds__(kBlock) k_neigh(NeighArgs a)
                         break;
                     }
                 if (found < 0)
-                    for (int oe2 = ob + kOld; oe2 < oe; oe2++) {
-                        const uint32_t ow = a.onj[oe2];
+                    for (int k = kOld; k < orow.cnt; k++) {
+                        const uint32_t ow = a.onj[orow.entry(k)];
                         if ((ow & (kFlagBit | kBondBit)) && a.otag[ow & kJMask] == tq) {
-                            found = oe2 - ob;
+                            found = k;
                             break;
                         }
                     }
+                if (found >= 0) found = orow.entry(found);
             }
             if (STAGE && pass) {   // kFlagBit marks a touching entry here
                 const int k = written + __popcll(m & ((1ull << lane) - 1ull));
                 const uint32_t w = (uint32_t)q | ((uint32_t)qcode << 26) | (touch ? kFlagBit : 0u);
                 if (k < kStageSlots)
-                    a.stage[(size_t)p * kStageSlots + k] = make_int2((int)w, found >= 0 ? ob + found : -1);
+                    a.stage[(size_t)p * kStageSlots + k] = make_int2((int)w, found);
             }
             if (FILL && emit) {
                 const int e = ebase + written + __popcll(m & ((1ull << lane) - 1ull));
                 uint32_t w = (uint32_t)q | ((uint32_t)qcode << 26);
                 if (found >= 0) {
-                    copy_hist(a.hist + (size_t)e * a.dnum, a.ohist + (size_t)(ob + found) * a.dnum, a.dnum);
-                    w |= a.onj[ob + found] & (kFlagBit | kBondBit);
+                    copy_hist(a.hist + (size_t)e * a.dnum, a.ohist + (size_t)found * a.dnum, a.dnum);
+                    w |= a.onj[found] & (kFlagBit | kBondBit);
                 } else if (a.coh_off >= 0) {
                     // the cohesion model reads its slots on entries that
                     // never touched (bond creation), so they start at zero
@@ -558,6 +559,8 @@ __global__ void __launch_bounds__(kBlock) k_neigh(NeighArgs a)
             }
         }
         written += __popcll(m);
+        if (!FILL) wtouch += __popcll((__ballot(emit && touch) & gmask) >> gshift);
+    }
     }
     // the staging row's last 64-byte granule written whole (a partial
     // granule costs a read-modify-write in HBM)
@@ -565,7 +568,10 @@ __global__ void __launch_bounds__(kBlock) k_neigh(NeighArgs a)
         const int k = written + lane;
         if (k < kStageSlots && k < ((written + 7) & ~7)) a.stage[(size_t)p * kStageSlots + k] = make_int2(0, -1);
     }
-    if (!FILL && lane == 0) a.count[p] = written;
+    if (!FILL && lane == 0) {
+        a.count[p] = wtouch;
+        a.count[a.n + p] = written - wtouch;
+    }
 }
 
 // The staged rows into the list, once the row lengths are scanned: G lanes
@@ -591,14 +597,14 @@ __global__ void __launch_bounds__(kBlock) k_neigh_compact(NeighArgs a)
     const int p = (blockIdx.x * blockDim.x + threadIdx.x) / G;
     if (p >= a.n) return;  // uniform across the group
     if (*a.maxcount > kStageSlots) return;
-    if ((int64_t)a.nstart[a.n] > a.ecap) {
+    if ((int64_t)a.nstart[2 * a.n] > a.ecap) {
         if (lane == 0) atomicOr(a.err, 8);
         return;
     }
     const int2 *row = a.stage + (size_t)p * kStageSlots;
     const int2 st0 = row[lane];   // inside the staging row, whatever cnt is
-    const int e0 = a.nstart[p];
-    const int cnt = a.nstart[p + 1] - e0;
+    const Row nr = list_row(a.nstart, a.n, p);
+    const int cnt = nr.cnt;
     const int2 st1 = cnt > G ? row[lane + G] : make_int2(0, -1);   // rows past G entries are rare
     const bool v0 = lane < cnt, v1 = lane + G < cnt;
     const bool tc0 = v0 && ((uint32_t)st0.x & kFlagBit), tc1 = v1 && ((uint32_t)st1.x & kFlagBit);
@@ -610,11 +616,11 @@ __global__ void __launch_bounds__(kBlock) k_neigh_compact(NeighArgs a)
     const int d0 = tc0 ? __popc(mt0 & below) : nt + __popc(mn0 & below);
     const int d1 = tc1 ? __popc(mt0) + __popc(mt1 & below) : nt + __popc(mn0) + __popc(mn1 & below);
     if (v0) {
-        a.nj[e0 + d0] = ((uint32_t)st0.x & ~kFlagBit) | (st0.y >= 0 ? a.onj[st0.y] & (kFlagBit | kBondBit) : 0u);
+        a.nj[nr.entry(d0)] = ((uint32_t)st0.x & ~kFlagBit) | (st0.y >= 0 ? a.onj[st0.y] & (kFlagBit | kBondBit) : 0u);
         s_src[grp][d0] = st0.y;
     }
     if (v1) {
-        a.nj[e0 + d1] = ((uint32_t)st1.x & ~kFlagBit) | (st1.y >= 0 ? a.onj[st1.y] & (kFlagBit | kBondBit) : 0u);
+        a.nj[nr.entry(d1)] = ((uint32_t)st1.x & ~kFlagBit) | (st1.y >= 0 ? a.onj[st1.y] & (kFlagBit | kBondBit) : 0u);
         s_src[grp][d1] = st1.y;
     }
     __builtin_amdgcn_wave_barrier();
@@ -626,11 +632,11 @@ __global__ void __launch_bounds__(kBlock) k_neigh_compact(NeighArgs a)
     // entries after it have flag 0, and an unflagged entry's history is not
     // read (a first contact starts from zero), so it is left unwritten,
     // except that the cohesion models read their slots on every entry
-    const int H = (a.coh_off >= 0 ? cnt : nt) * dnum;   // <= kStageSlots * dnum < 2^11
+    const int H = nt * dnum;   // <= kStageSlots * dnum < 2^11
     // t / dnum as (t * inv) >> 20: exact for t < 2^11, dnum <= 64
     const uint32_t inv = (1u << 20) / (uint32_t)dnum + 1u;
     const double *__restrict__ oh = a.ohist;
-    double *__restrict__ hb = a.hist + (size_t)e0 * dnum;
+    double *__restrict__ hb = a.hist + (size_t)nr.a0 * dnum;
     for (int t0 = 0; t0 < H; t0 += U * G) {
         double v[U];
 #pragma unroll
@@ -648,6 +654,10 @@ __global__ void __launch_bounds__(kBlock) k_neigh_compact(NeighArgs a)
             if (t < H) hb[t] = v[u];
         }
     }
+    if (a.coh_off >= 0) {
+        double *__restrict__ hn = a.hist + (size_t)nr.b0 * dnum;
+        for (int t = lane; t < (cnt - nt) * dnum; t += G) hn[t] = 0.0;
+    }
 }
 
 // Longest row, for the neigh_modify one check: a grid-stride max over the
@@ -655,11 +665,12 @@ __global__ void __launch_bounds__(kBlock) k_neigh_compact(NeighArgs a)
 // serialises a million times per rebuild).
 constexpr int kMaxBlocks = 512;
 
-__global__ void __launch_bounds__(kBlock) k_row_max(const int *count, int n, int *maxcount)
+__global__ void __launch_bounds__(kBlock) k_row_max(const int *count, int n, int parts, int *maxcount)
 {
     __shared__ int s_m[kBlock / 64];
     int m = 0;
-    for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) m = max(m, count[i]);
+    for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock)
+        m = max(m, count[i] + (parts == 2 ? count[n + i] : 0));
     for (int o = 32; o > 0; o >>= 1) m = max(m, __shfl_xor(m, o, 64));
     if ((threadIdx.x & 63) == 0) s_m[threadIdx.x >> 6] = m;
     __syncthreads();
@@ -708,7 +719,7 @@ void launch_neigh_count(const NeighArgs &a, hipStream_t s)
     case 8: launch_search<kCount, 8>(a, s); break;
     default: launch_search<kCount, 16>(a, s); break;
     }
-    launch_row_max(a.count, a.n, a.maxcount, s);
+    launch_row_max(a.count, a.n, 2, a.maxcount, s);
 }
 
 void launch_neigh_stage(const NeighArgs &a, hipStream_t s)
@@ -720,7 +731,7 @@ void launch_neigh_stage(const NeighArgs &a, hipStream_t s)
     case 8: launch_search<kStage, 8>(a, s); break;
     default: launch_search<kStage, 16>(a, s); break;
     }
-    launch_row_max(a.count, a.n, a.maxcount, s);
+    launch_row_max(a.count, a.n, 2, a.maxcount, s);
 }
 
 void launch_neigh_compact(const NeighArgs &a, hipStream_t s)
@@ -730,11 +741,11 @@ void launch_neigh_compact(const NeighArgs &a, hipStream_t s)
     k_neigh_compact<G><<<group_blocks(a.n, G), kBlock, 0, s>>>(a);
 }
 
-void launch_row_max(const int *count, int n, int *maxcount, hipStream_t s)
+void launch_row_max(const int *count, int n, int parts, int *maxcount, hipStream_t s)
 {
     if (n == 0) return;
     const int nb = (int)std::min<long long>(kMaxBlocks, ((long long)n + kBlock - 1) / kBlock);
-    k_row_max<<<nb, kBlock, 0, s>>>(count, n, maxcount);
+    k_row_max<<<nb, kBlock, 0, s>>>(count, n, parts, maxcount);
 }
 
 void launch_neigh_fill(const NeighArgs &a, hipStream_t s)

@@ -1,0 +1,66 @@
+"""The tiled contact pass at its edges (MI355X), against the oracle.
+
+A lattice of spheres that do not touch at the build, with a skin that lists
+tens of partners per sphere, contracts until every neighbour touches, without a
+rebuild: all contacts then come from the rows' second part, so a tile's queue
+overflows into full batches, its entry map (16 per particle) runs out, and the
+first range is empty.  A second run rebuilds on the way, so both ranges are in
+use.  Sizes leave tiles of one, of all but one and of every particle, for
+every tile width and history layout.
+"""
+import numpy as np
+import pytest
+
+from conftest import load_engine
+from oracle import Oracle
+from test_gpu_parity import HYST, check_forces, check_pairs
+
+pytestmark = pytest.mark.gpu
+
+
+def contracting(n, skin, rolling, normal, every):
+    rng = np.random.default_rng(n)
+    r0, gap = 1e-3, 2.004e-3
+    side = int(np.ceil(n ** (1 / 3)))
+    g = np.stack(np.meshgrid(*[np.arange(side)] * 3, indexing="ij"), -1).reshape(-1, 3)[:n]
+    x = 0.02 + gap * g + rng.uniform(-1e-6, 1e-6, (n, 3))
+    r = np.full(n, r0)
+    W = load_engine().workloads
+    mats = W._materials(mur=0.1, etar=0.3)
+    if normal != "hertz":
+        mats["hysteretic"] = HYST
+    spec = dict(box_lo=[0.0] * 3, box_hi=[0.06] * 3, periodic=[0, 0, 0], dt=1e-6, skin=skin, cdf=1.0,
+                neigh_every=every, neigh_delay=0, neigh_check=False, rolling=rolling, normal=normal,
+                wall_normal="hertz", materials=mats, planes=[(2, 0.0, 1)], gravity=(0.0, 0.0, -9.81))
+    atoms = dict(x=x, v=-60.0 * (x - x.mean(0)), omega=rng.uniform(-20, 20, (n, 3)), radius=r,
+                 rmass=4.0 / 3.0 * np.pi * r ** 3 * 2500.0, type=np.ones(n, np.int32),
+                 tag=np.arange(1, n + 1, dtype=np.int32))
+    return spec, atoms
+
+
+@pytest.mark.parametrize("rolling,normal", [("off", "hertz"), ("epsd", "hertz"), ("epsd", "hysteretic/nonlinear1"),
+                                            ("off", "hysteretic/nonlinear1")])
+@pytest.mark.parametrize("every", [1000, 10])
+def test_tiles_at_their_edges(rolling, normal, every):
+    eng = load_engine()
+    for n, skin in ((1, 2e-3), (9, 2e-3), (63, 2.2e-3), (65, 2.2e-3), (343, 2.2e-3)):
+        spec, atoms = contracting(n, skin, rolling, normal, every)
+        o = Oracle(spec, atoms)
+        o.setup()
+        o.run(60)
+        for tile in (-8, -16, -32, -64):
+            for precision in ("fp64", "mixed") if normal == "hertz" else ("fp64",):
+                s = eng.Simulation(spec, atoms, precision=precision)
+                s.set_contact_shape(tile, 64 if tile != -16 else 256)
+                s.setup()
+                s.step(60)
+                # 60 steps of rounding, as the parity tests bound a short
+                # horizon; the mixed law's 1e-7 grows like it
+                if n > 1:
+                    check_forces(s, o, 1e-9 if precision == "fp64" else 1e-4)
+                    if precision == "fp64":
+                        check_pairs(s, o, hist_tol=1e-9)
+                s.close()
+        if n == 343:
+            touching = (np.asarray(o.pairs()[4]) != 0).sum()
+            assert touching >= 2 * 3 * 7 * 7 * 6, touching   # every lattice neighbour, both ways
