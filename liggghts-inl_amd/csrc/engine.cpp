@@ -2858,31 +2858,45 @@ extern "C" int dem_step(dem_ctx *ctx, int nsteps)
     return check_err_flag(ctx);
 }
 
+// The vectors in upload order: permuted on the device, then copied straight
+// into the caller's arrays.  The permuted arrays (120 B per particle) use the
+// rebuild's staging rows (256 B), which hold nothing between rebuilds.
 extern "C" int dem_download(dem_ctx *ctx, double *x, double *v, double *omega, double *f, double *torque)
 {
     if (!ctx) return fail(nullptr, DEM_ERR_ARG, "null context");
     sync_enter(ctx);
-    const int n = ctx->n, c = ctx->cur;
+    const int n = ctx->n;
     if (n == 0) return DEM_OK;
-    std::vector<double4> hx(n), hv(n), hw(n), hf(n), ht(n);
-    std::vector<int> ho(n);
-    HIPCHK(hipStreamSynchronize(ctx->stream));
-    HIPCHK(hipMemcpy(ho.data(), ctx->orig[c], n * sizeof(int), hipMemcpyDeviceToHost));
-    HIPCHK(hipMemcpy(hx.data(), sx(ctx), n * sizeof(double4), hipMemcpyDeviceToHost));
-    HIPCHK(hipMemcpy(hv.data(), sv(ctx), n * sizeof(double4), hipMemcpyDeviceToHost));
-    HIPCHK(hipMemcpy(hw.data(), sw(ctx), n * sizeof(double4), hipMemcpyDeviceToHost));
-    HIPCHK(hipMemcpy(hf.data(), ctx->f4, n * sizeof(double4), hipMemcpyDeviceToHost));
-    HIPCHK(hipMemcpy(ht.data(), ctx->t4, n * sizeof(double4), hipMemcpyDeviceToHost));
-    auto put = [&](double *dst, const std::vector<double4> &src) {
-        if (!dst) return;
-        for (int i = 0; i < n; i++) {
-            const int o = ho[i];
-            dst[3 * o] = src[i].x;
-            dst[3 * o + 1] = src[i].y;
-            dst[3 * o + 2] = src[i].z;
+    static_assert(kStageSlots * sizeof(int2) >= 15 * sizeof(double), "five vectors fit the staging rows");
+    hipStream_t s = ctx->stream;
+    const double4 *src[5] = {sx(ctx), sv(ctx), sw(ctx), ctx->f4, ctx->t4};
+    double *dst[5] = {x, v, omega, f, torque};
+    UnsortArgs ua{};
+    ua.orig = ctx->orig[ctx->cur];
+    ua.out = reinterpret_cast<double *>(ctx->stage);
+    ua.n = n;
+    int nv = 0;
+    for (int k = 0; k < 5; k++)
+        if (dst[k]) {
+            dst[nv] = dst[k];
+            ua.v[nv++] = src[k];
         }
-    };
-    put(x, hx); put(v, hv); put(omega, hw); put(f, hf); put(torque, ht);
+    if (nv == 0) return DEM_OK;
+    launch_unsort(ua, nv, s);
+    KCHK();
+    const size_t b = 3 * (size_t)n * sizeof(double);
+    // each copy is a round trip of its own: a few particles go over in one
+    constexpr int kOneCopy = 8192;
+    if (n <= kOneCopy) {
+        std::vector<double> h(3 * (size_t)n * nv);
+        HIPCHK(hipMemcpyAsync(h.data(), ua.out, b * nv, hipMemcpyDeviceToHost, s));
+        HIPCHK(hipStreamSynchronize(s));
+        for (int k = 0; k < nv; k++) memcpy(dst[k], h.data() + 3 * (size_t)n * k, b);
+        return DEM_OK;
+    }
+    for (int k = 0; k < nv; k++)
+        HIPCHK(hipMemcpyAsync(dst[k], ua.out + 3 * (size_t)n * k, b, hipMemcpyDeviceToHost, s));
+    HIPCHK(hipStreamSynchronize(s));
     return DEM_OK;
 }
 

@@ -329,6 +329,14 @@ void launch_fill_int(int *p, int v, int n, hipStream_t s);
 void launch_cap_guard(int *nstart, int n, int64_t ecap, int *flag, int *err, int bit, hipStream_t s);
 void launch_row_max_check(const int *maxcount, int limit, int *err, int bit, hipStream_t s);
 void launch_copy_int(int *dst, const int *src, int n, hipStream_t s);
+// out[3 (n k + orig[i]) ..] = v[k][i].xyz for nv <= 5 vectors
+struct UnsortArgs {
+    const double4 *v[5];
+    const int *orig;
+    double *out;
+    int n;
+};
+void launch_unsort(const UnsortArgs &a, int nv, hipStream_t s);
 // out[b*5 + {0..4}] = count, sum z, sum of pwf, sum mass, kinetic energy of
 // instance b (particles in key order)
 void launch_inst_obs(const int *cstart, int nkl, int ninst, const double4 *xr, const double4 *vm,
