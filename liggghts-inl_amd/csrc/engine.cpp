@@ -212,6 +212,7 @@ struct dem_ctx {
     bool fold = false;
     int fold_par = 0;
     bool cg_fold = false;
+    int check_interval = 0;   // steps between the last two rebuilds that a distance check asked for
     double *d_gpart = nullptr, *d_gtot = nullptr;   // partial sums; 4 per op slot
     int ago = 0;
 
@@ -1329,6 +1330,14 @@ static int force_pass(dem_ctx *ctx, int shearupdate, int integ = 0)
         fa.dtf = 0.5 * ctx->p.dt;   // as in integrate()
         fa.dtv = ctx->p.dt;
         fa.dtfrotate = fa.dtf / 0.4;
+        if (ctx->fold && integ == 3) {
+            fa.ctl = ctx->ctl;
+            fa.par = ctx->fold_par;
+            fa.xhold = ctx->xhold;
+            const double trig = 0.5 * ctx->p.skin;   // as decide() squares it
+            fa.deltasq = trig * trig;
+            fa.halt = nullptr;
+        }
     }
     if (ctx->M.cohesion != CM_OFF) {
         BondArgs ba{};
@@ -2605,7 +2614,7 @@ static int capture_graph(dem_ctx *ctx)
 
 static bool checked_graph_ok(const dem_ctx *ctx)
 {
-    if (!ctx->use_graph || ctx->window || !ctx->fops.empty() || !ctx->moves.empty() || !ctx->p.neigh_check
+    if (ctx->window || !ctx->fops.empty() || !ctx->moves.empty() || !ctx->p.neigh_check
         || ctx->p.neigh_every != 1 || ctx->p.neigh_delay != 0 || ctx->mf.mesh >= 0 || ctx->timing || ctx->n == 0
         || ctx->tape_pos >= 0)
         return false;
@@ -2635,29 +2644,26 @@ static std::vector<const void *> checked_key(const dem_ctx *ctx)
     return k;
 }
 
-// Record P steps (P even), each: the distance check (which also advances
-// the step counter), the force pass with final_integrate(n) +
-// initial_integrate(n+1), the mesh move.  When the integrator has its own
-// pass (no fused integration) that pass does the next step's check and the
-// mesh moves instead (two launches fewer per step).
-static int capture_checked_graph(dem_ctx *ctx, int P)
+// Whether a checked period's own passes do the next step's check (and the mesh
+// moves): the integrator's pass, or the contact pass that integrates when
+// nothing moves beside the particles.  Two launches fewer per step, one fewer.
+static bool checked_fold(const dem_ctx *ctx)
 {
     int nmoving = 0;
     for (const auto &m : ctx->meshes) nmoving += m.moving ? 1 : 0;
-    const bool fold = !fuse_possible(ctx) && nmoving <= kFoldMeshes;
-    if (ctx->cgexec) {
-        HIPCHK(hipGraphExecDestroy(ctx->cgexec));
-        ctx->cgexec = nullptr;
-    }
-    if (!ctx->ctl && dev_alloc(ctx, &ctx->ctl, 3)) return DEM_ERR_HIP;
-    HIPCHK(hipStreamSynchronize(ctx->stream));
-    const int cur0 = ctx->cur, lcur0 = ctx->lcur, par0 = ctx->par;
+    if (!fuse_possible(ctx)) return nmoving <= kFoldMeshes;
+    return last_wall_mesh(ctx) < 0 && nmoving == 0;
+}
+
+// P steps (P even) on the stream, each: the distance check (which also
+// advances the step counter), the force pass with final_integrate(n) +
+// initial_integrate(n+1), the mesh move; folded periods check each next step
+// at the end of the step before.  flip: whether a step swaps the state buffers.
+static int checked_steps(dem_ctx *ctx, int P, bool fold, int *flip)
+{
     const double trig = 0.5 * ctx->p.skin;
-    hipGraph_t graph = nullptr;
-    HIPCHK(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
-    ctx->gexec_capturing = true;
     ctx->halt_dev = ctx->ctl + 2;
-    int rc = DEM_OK, flip = 0;
+    int rc = DEM_OK;
     for (int k = 0; k < P && rc == DEM_OK; k++) {
         ctx->step_dev = ctx->ctl + (k & 1);
         if (!fold) launch_check_halt(sx(ctx), ctx->xhold, ctx->n, trig * trig, ctx->ctl, k & 1, ctx->stream);
@@ -2666,12 +2672,29 @@ static int capture_checked_graph(dem_ctx *ctx, int P)
         ctx->fold_par = k & 1;
         rc = force_pass(ctx, 1, 3);
         ctx->fold = false;
-        if (k == 0) flip = ctx->par != pb;
+        if (k == 0) *flip = ctx->par != pb;
         if (rc == DEM_OK && !fold) rc = move_meshes(ctx);
     }
     ctx->halt_dev = nullptr;
     ctx->step_dev = nullptr;
-    ctx->fold = false;
+    return rc;
+}
+
+// Record P such steps into a graph.
+static int capture_checked_graph(dem_ctx *ctx, int P)
+{
+    const bool fold = checked_fold(ctx);
+    if (ctx->cgexec) {
+        HIPCHK(hipGraphExecDestroy(ctx->cgexec));
+        ctx->cgexec = nullptr;
+    }
+    HIPCHK(hipStreamSynchronize(ctx->stream));
+    const int cur0 = ctx->cur, lcur0 = ctx->lcur, par0 = ctx->par;
+    hipGraph_t graph = nullptr;
+    HIPCHK(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
+    ctx->gexec_capturing = true;
+    int flip = 0;
+    const int rc = checked_steps(ctx, P, fold, &flip);
     ctx->gexec_capturing = false;
     const hipError_t ec = hipStreamEndCapture(ctx->stream, &graph);
     const bool same_par = ctx->par == par0;
@@ -2733,20 +2756,31 @@ static long long mesh_horizon(const dem_ctx *ctx, long long room)
 
 // Whole checked periods from iteration st (step ntimestep + 1) on, at most
 // up to the step before the last, the next insertion or forced rebuild.
-// Advances st and ntimestep by the steps that completed.
-static int checked_periods(dem_ctx *ctx, int nsteps, int &st)
+// Advances st and ntimestep by the steps that completed; again: all of them
+// did, and no check asked for a rebuild.
+//
+// How many go out before the host looks: steps launched past a halt return at
+// once, but cost a launch each, and a look costs a round trip (20 us).  The
+// last interval between rebuilds foresees the next: most of it at once, then
+// one period at a time around its end, then as many steps as it is overdue.
+static int checked_periods(dem_ctx *ctx, int nsteps, int &st, bool *again)
 {
+    *again = false;
     constexpr int P = 16;
     constexpr long long kMaxRun = 64 * P;   // steps per host read-back
     long long room = (long long)(nsteps - 1) - st;
     room = std::min(room, next_insert_step(ctx) - 1 - ctx->ntimestep);
     if (ctx->next_reneighbor > ctx->ntimestep) room = std::min(room, ctx->next_reneighbor - 1 - ctx->ntimestep);
-    room = std::min(room, kMaxRun);
+    const long long expect = (long long)ctx->check_interval * 7 / 8, ago = ctx->ago;
+    const long long run = ago < expect ? expect - ago : std::max<long long>(ago - ctx->check_interval, 0);
+    room = std::min(room, std::min(kMaxRun, std::max<long long>((run + P - 1) / P * P, P)));
     if (room < P) return DEM_OK;
     room = mesh_horizon(ctx, room);
     const long long R = room / P;
     if (R < 1) return DEM_OK;
-    if (!ctx->cgexec || ctx->cg_key != checked_key(ctx)) {
+    if (!ctx->ctl && dev_alloc(ctx, &ctx->ctl, 3)) return DEM_ERR_HIP;
+    const bool graph = ctx->use_graph;
+    if (graph && (!ctx->cgexec || ctx->cg_key != checked_key(ctx))) {
         const int rc = capture_checked_graph(ctx, P);
         if (rc) return rc;
     }
@@ -2757,16 +2791,29 @@ static int checked_periods(dem_ctx *ctx, int nsteps, int &st)
     HIPCHK(hipMemcpyAsync(ctx->ctl, ctx->ctl_h, sizeof(ctx->ctl_h), hipMemcpyHostToDevice, ctx->stream));
     // a folded period checks each next step at the end of the step before:
     // the first step's check runs here
-    if (ctx->cg_fold) {
+    const bool fold = graph ? ctx->cg_fold : checked_fold(ctx);
+    if (fold) {
         const double trig = 0.5 * ctx->p.skin;
         launch_check_halt(sx(ctx), ctx->xhold, ctx->n, trig * trig, ctx->ctl, 0, ctx->stream);
         KCHK();
     }
-    for (long long r = 0; r < R; r++) HIPCHK(hipGraphLaunch(ctx->cgexec, ctx->stream));
+    int flip = graph ? ctx->cg_flip : 0;
+    const int par0 = ctx->par;
+    ctx->gexec_capturing = true;   // timers and host copies stay out of the steps, as when recording
+    int rc = DEM_OK;
+    for (long long r = 0; r < R && rc == DEM_OK; r++) {
+        if (!graph) rc = checked_steps(ctx, P, fold, &flip);
+        else if (hipGraphLaunch(ctx->cgexec, ctx->stream) != hipSuccess)
+            rc = fail(ctx, DEM_ERR_HIP, "checked graph: launch failed");
+    }
+    ctx->gexec_capturing = false;
+    ctx->par = par0;
+    if (rc) return rc;
     HIPCHK(hipMemcpyAsync(ctx->ctl_h, ctx->ctl, sizeof(ctx->ctl_h), hipMemcpyDeviceToHost, ctx->stream));
     HIPCHK(hipStreamSynchronize(ctx->stream));
     const long long halt = ctx->ctl_h[2];
-    const long long done = halt ? halt - t0 - 1 : R * P;
+    // a halt past the last launched step is the next step's, which asks again
+    const long long done = halt ? std::min(halt - t0 - 1, R * P) : R * P;
     // the host side of each completed step: Neighbor::decide's count, the
     // mesh trigger (foreseen: it can fire on the last one only), the mesh move
     for (long long k = 0; k < done; k++) {
@@ -2775,8 +2822,9 @@ static int checked_periods(dem_ctx *ctx, int nsteps, int &st)
         mesh_trigger(ctx);
         move_meshes_host(ctx);
     }
-    if (ctx->cg_flip && (done & 1)) ctx->par ^= 1;
+    if (flip && (done & 1)) ctx->par ^= 1;
     st += (int)done;
+    *again = halt == 0;
     return DEM_OK;
 }
 
@@ -2793,7 +2841,9 @@ extern "C" int dem_step(dem_ctx *ctx, int nsteps)
     for (int st = 0; st < nsteps; st++) {
         if (cgok && st >= 1 && !split_prev && ctx->ntimestep + 1 != ctx->next_reneighbor
             && ctx->ntimestep > ctx->rel_until) {
-            if ((rc = checked_periods(ctx, nsteps, st))) return rc;
+            bool again = true;
+            while (again)
+                if ((rc = checked_periods(ctx, nsteps, st, &again))) return rc;
         }
         // whole graph periods while they fit before the last step, starting
         // right after a rebuild
@@ -2830,6 +2880,7 @@ extern "C" int dem_step(dem_ctx *ctx, int nsteps)
         // pre_exchange (fix insert) before the build, as Verlet::run
         // (verlet.cpp:304-327)
         if (nflag && !ctx->inserts.empty() && (rc = run_inserts(ctx))) return rc;
+        if (nflag && ctx->p.neigh_check) ctx->check_interval = ctx->ago;
         if (nflag && ctx->n > 0 && (rc = ctx->window ? window_mask(ctx) : rebuild(ctx))) return rc;
         if (!nflag) mesh_trigger(ctx);
         if (ctx->tape_pos >= 0 && (rc = tape_store(ctx, nflag))) return rc;

@@ -208,14 +208,35 @@ __device__ inline void integrate_into(const ForceArgs &a, int i, double4 x, doub
     a.xn[i] = x;
     a.vn[i] = v;
     a.wn[i] = w;
+    if (a.ctl) {   // Neighbor::check_distance of the next step
+        const double4 b = a.xhold[i];
+        const double dx = x.x - b.x, dy = x.y - b.y, dz = x.z - b.z;
+        const long long step = a.ctl[a.par];
+        if (dx * dx + dy * dy + dz * dz > a.deltasq)
+            atomicCAS((unsigned long long *)&a.ctl[2], 0ull, (unsigned long long)(step + 1));
+        if (i == 0) a.ctl[a.par ^ 1] = step + 1;
+    }
+}
+
+// Whether this step of a checked period still runs: not once the period
+// halted at or before it.  A halt that the pass records itself names the next
+// step, so blocks that start after it still run.  The counter advances either
+// way (from the pass's first particle).
+__device__ inline bool period_runs(const ForceArgs &a, bool first)
+{
+    if (!a.ctl) return !(a.halt && *a.halt);
+    const long long step = a.ctl[a.par], h = a.ctl[2];
+    if (h == 0 || h > step) return true;
+    if (first) a.ctl[a.par ^ 1] = step + 1;
+    return false;
 }
 
 template <bool MIXED, int G, int NM, int WN, bool CH = false>
 __global__ void __launch_bounds__(kBlock) k_force(ForceArgs a)
 {
-    if (a.halt && *a.halt) return;
     const int blk = xcd_block(blockIdx.x, gridDim.x);
     const int tid = blk * blockDim.x + threadIdx.x;
+    if (!period_runs(a, tid == 0)) return;
     const int g = threadIdx.x & (G - 1);
     const int i = tid / G;
     const bool live = i < a.n;      // dead groups still join the shuffles
@@ -441,7 +462,7 @@ __global__ void __launch_bounds__(kBlock) k_force_t(ForceArgs a)
     const int blk = xcd_block(blockIdx.x, gridDim.x);
     const int p0 = (blk * (int)(blockDim.x >> 6) + wv) * P;
     if (p0 >= a.n) return;   // uniform over the wave
-    if (a.halt && *a.halt) return;
+    if (!period_runs(a, p0 == 0 && lane == 0)) return;
     Lds &L = reinterpret_cast<Lds *>(s_raw)[wv];
     const int np = min(P, a.n - p0);
     const Model &M = a.M;

@@ -36,6 +36,12 @@ struct ForceArgs {
     // a checked graph period: nonzero *halt (the step whose distance check
     // asked for a rebuild) makes the pass return at once; null: always run
     const long long *halt;
+    // a checked period whose contact pass integrates (fuse = 3) also checks
+    // the next step's positions there (as IntegArgs::ctl; then halt is null)
+    long long *ctl;
+    int par;
+    const double4 *xhold;
+    double deltasq;
     Model M;
     Planes P;
 };
