@@ -40,6 +40,23 @@ struct NormalOut {
     double Fn, kn, kt, gammat;
 };
 
+// The reference's pow(z, 2), pow(z, 0.5) and pow(z, +-0.25) of the hysteretic
+// laws without the device's general pow, which is several hundred
+// instructions, two to four calls per contact.  The square and the root are
+// correctly rounded operations; root4 adds the first-order rest of its two
+// roots (from their residuals, exact in an fma) to the rounded ones: largest
+// error 0.50 ulp (the pow 1.00) over 1e-13..20.  Contact pass of a 100,000-
+// sphere hysteretic/nonlinear1 column: 70 -> 55 us, with no change in registers.
+template <bool INVERSE>
+__device__ inline double root4(double z)
+{
+    const double s = sqrt(z), y = sqrt(s), i = 1. / y;
+    if (!(z > 0. && i > 0.)) return INVERSE ? i : y;   // 0, infinity, NaN
+    const double rest = 0.5 * i * fma(0.5 * i * i, fma(-s, s, z), fma(-y, y, s));
+    return INVERSE ? fma(i, fma(-y, i, 1.) - i * rest, i) : y + rest;
+}
+__device__ inline double pow2(double z) { return z * z; }
+
 // NormalModel<HYSTERETIC_NONLINEAR1/2>::surfacesIntersect; writes its
 // twelve history slots whatever shearupdate says, and sqrt(5/4) is the
 // reference's integer expression, sqrt(1) = 1.
@@ -98,10 +115,10 @@ __device__ inline NormalOut normal_hysteretic(const double *mat, const ContactIn
             else if (deltan <= deltaMin) fHys = -k_c * deltan;
             else fHys = betan * (deltan - deltaZero);
         } else {
-            fHys = Alpha_in * k1 * pow(deltan - deltaZero, 2) + f0;
+            fHys = Alpha_in * k1 * pow2(deltan - deltaZero) + f0;
         }
-        const double pw = (NM == NM_HYST2) ? 0.5 : 0.25;
-        gamman = sqrt54 * sqrt(4. * meff * Alpha_in * k1 / dampfac) * (pow(deltan, pw) + pow(deltaZero, pw));
+        const double pw = (NM == NM_HYST2) ? sqrt(deltan) + sqrt(deltaZero) : root4<false>(deltan) + root4<false>(deltaZero);
+        gamman = sqrt54 * sqrt(4. * meff * Alpha_in * k1 / dampfac) * pw;
         gammat = gamman;
         history[1] = deltaZero;
         history[2] = k1;
@@ -116,14 +133,14 @@ __device__ inline NormalOut normal_hysteretic(const double *mat, const ContactIn
         if (NM == NM_HYST1) {
             k2 = A3_in * k1_old;
             deltaZero = (1 - k1_old / k2) * deltaMax;
-            const double beta = Alpha_in * k1_old * pow(deltaMax - deltaZero_old, 2) / k2 / (deltaMax - deltaZero);
+            const double beta = Alpha_in * k1_old * pow2(deltaMax - deltaZero_old) / k2 / (deltaMax - deltaZero);
             deltaMin = beta * (k2 - k1_old) / (beta * k2 + k_c) * deltaMax;
             k1 = deltaMax * A1_in + A2_in;
             if (deltan >= deltaMin) {
                 betan = beta * k2;
                 if (deltan >= deltaZero) {
                     fHys = beta * k2 * (deltan - deltaZero) + (deltan - deltaZero) * f0_old / (deltaMax - deltaZero);
-                    f0 = fHys - Alpha_in * k1 * pow(deltan - deltaZero, 2);
+                    f0 = fHys - Alpha_in * k1 * pow2(deltan - deltaZero);
                 } else {
                     fHys = beta * k2 * (deltan - deltaZero);
                     f0 = 0;
@@ -132,24 +149,24 @@ __device__ inline NormalOut normal_hysteretic(const double *mat, const ContactIn
                 fHys = -k_c * deltan;
                 f0 = 0;
             }
-            gamman = sqrt54 * sqrt(4. * meff * Alpha_in * k1_old / dampfac) * (pow(deltan, 0.25));
+            gamman = sqrt54 * sqrt(4. * meff * Alpha_in * k1_old / dampfac) * root4<false>(deltan);
         } else {
             k2 = A3_in * (A1_in * deltaMax + A2_in);
             deltaZero = fcc * (1 - k1_old / k2) * deltaMax;
             deltaZero_old = history[3];
-            betan = log(Alpha_in * k1_old / Cin_in / k2 * pow(deltaMax - deltaZero_old, 2) + 1)
+            betan = log(Alpha_in * k1_old / Cin_in / k2 * pow2(deltaMax - deltaZero_old) + 1)
                     / (deltaMax - fcc * (1 - k1_old / k2) * deltaMax);
             deltaMin = betan * (k2 - k1_old) / (betan * k2 + k_c) * deltaMax;
             k1 = deltaMax * A1_in + A2_in;
             if (deltan >= deltaZero) {
                 fHys = Cin_in * k2 * (exp(betan * (deltan - deltaZero)) - 1)
                        + (deltan - deltaZero) * f0_old / (deltaMax - deltaZero);
-                f0 = fHys - Alpha_in * k1 * pow(deltan - deltaZero, 2);
+                f0 = fHys - Alpha_in * k1 * pow2(deltan - deltaZero);
             } else {
                 fHys = Cin_in * k2 * (exp(betan * (deltan - deltaZero)) - 1);
                 f0 = 0;
             }
-            gamman = 1 * 0.001 * sqrt54 * sqrt(4. * meff * Alpha_in * k1_old / dampfac) * (pow(deltan, -0.25));
+            gamman = 1 * 0.001 * sqrt54 * sqrt(4. * meff * Alpha_in * k1_old / dampfac) * root4<true>(deltan);
         }
         gammat = gamman;
         history[1] = deltaZero;

@@ -194,10 +194,10 @@ struct dem_ctx {
     double4 *rel[2] = {};
     long long rel_until = -1;
     int rel_mask = 0;
-    // checked graph periods (neigh_modify check yes): ctl[0], ctl[1] the
+    // checked periods (neigh_modify check yes): ctl[0], ctl[1] the
     // current step, alternately; ctl[2] the step whose distance check asked
-    // for a rebuild; while such a period is being recorded halt_dev = ctl + 2
-    // and step_dev = the recorded step's counter
+    // for a rebuild; while such a period is recorded or launched halt_dev =
+    // ctl + 2 and step_dev = the step's counter
     long long *ctl = nullptr;
     long long ctl_h[3] = {0, 0, 0};
     const long long *halt_dev = nullptr;
@@ -2602,14 +2602,15 @@ static int capture_graph(dem_ctx *ctx)
     return DEM_OK;
 }
 
-// ---- checked graph periods (neigh_modify check yes, every 1, delay 0)
+// ---- checked periods (neigh_modify check yes, every 1, delay 0)
 //
-// Neighbor::decide's distance check runs on the device inside the recorded
-// steps: the first step whose check asks for a rebuild halts the period (the
+// Neighbor::decide's distance check runs on the device inside the steps, which
+// are replayed from a graph under dem_use_graph and launched one by one
+// otherwise: the first step whose check asks for a rebuild halts the period (the
 // step's own kernels and every later one return at once), and the host,
 // reading the halt word once per batch of periods, goes on eagerly from that
 // step, whose check then asks again.  Rebuilds therefore never run inside
-// such a graph, and a moving mesh's trigger is foreseen on the host (its
+// such a period, and a moving mesh's trigger is foreseen on the host (its
 // motion is known), so no host round trip is needed per step.
 
 static bool checked_graph_ok(const dem_ctx *ctx)

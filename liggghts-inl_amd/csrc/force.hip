@@ -367,12 +367,12 @@ __global__ void __launch_bounds__(kBlock) k_force(ForceArgs a)
 // atomics, and a sum that does not depend on where the tiles begin.
 //
 // What bounds it: the latency of its chain of gathers at 4 (mixed) or 3
-// (FP64) waves per SIMD, which the 126 / 142 registers of the law allow, with
+// (FP64) waves per SIMD, which the 128 / 142 registers of the law allow, with
 // 48 % of the issue slots taken by VALU.  Of the 700 B per particle of HBM
 // traffic 195 + 195 are histories; with rows of touching and other partners
 // mixed (whole rows one after the other) it was 836 B, and every entry went
 // through the test and a queue.  1M-sphere column: 276 -> 231 us mixed, 282 ->
-// 248 FP64.  Slower here: histories and state through LDS in whole lines (249
+// 242 FP64.  Slower here: histories and state through LDS in whole lines (249
 // to 270 us), the first batch fetched ahead of the test (256, one wave per
 // SIMD fewer), tiles trimmed so that their batches fill (236).
 constexpr int kQueue = 192;   // 63 waiting and the 128 of one test

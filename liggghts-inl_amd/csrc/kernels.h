@@ -33,7 +33,7 @@ struct ForceArgs {
     // mixed law: the partners' velocity/mass and spin/meta as one 32-byte
     // FP32 record per particle (2 float4), or null to read vm/wt
     const float4 *rec;
-    // a checked graph period: nonzero *halt (the step whose distance check
+    // a checked period: nonzero *halt (the step whose distance check
     // asked for a rebuild) makes the pass return at once; null: always run
     const long long *halt;
     // a checked period whose contact pass integrates (fuse = 3) also checks
@@ -63,7 +63,7 @@ struct BondArgs {
     const double *brid;
     int n, shearupdate;
     long long ntimestep;
-    // in a checked graph period: the step counter on the device (read
+    // in a checked period: the step counter on the device (read
     // instead of ntimestep) and the halt word, as ForceArgs::halt
     const long long *step_dev;
     const long long *halt;
@@ -158,7 +158,7 @@ struct IntegArgs {
     double mv_delta;             // (step - time_origin) * dt of the initial half
     const double4 *xo;           // positions at the fix's creation
     const long long *halt;       // as ForceArgs::halt
-    // a checked graph period with the integrator in its own pass (mode 3):
+    // a checked period with the integrator in its own pass (mode 3):
     // ctl as in launch_check_halt; the pass runs unless the period halted
     // before this step, then checks the next step's positions (the next
     // step's decision) and moves up to kFoldMeshes meshes by their step
@@ -379,7 +379,7 @@ void launch_sum6(const double *v, int n, double *part, double *out, hipStream_t 
 int scan_tmp_size(int n);
 // Neighbor::check_distance (neighbor.cpp:1390-1465): flag |= 1 if any atom
 // moved more than sqrt(deltasq) since the last build.
-// A checked graph period keeps the current step in ctl[par] (par alternates
+// A checked period keeps the current step in ctl[par] (par alternates
 // over the recorded steps) and in ctl[2] the step whose distance check asked
 // for a rebuild (0: none yet).  k_check_halt, unless halted, writes the next
 // step to ctl[par ^ 1] and records the step when an atom moved more than
