@@ -30,10 +30,10 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 HBM_PEAK_GBS = 8000.0
 # HBM bytes per particle of one mixed contact pass (integrator fused, no force
 # output) on this workload, from the FETCH_SIZE and WRITE_SIZE counter passes
-# of rocprofv3 on k_force_q<true,32> (FETCH_SIZE scaled x2.0, WRITE_SIZE x1.0
+# of rocprofv3 on k_force_t<true,0,0,6,32> (FETCH_SIZE scaled x2.0, WRITE_SIZE x1.0
 # against a 256 MiB device copy), averaged over the stepping dispatches:
 # profiles/pmc_traffic_k_force_column1M.md.  Re-measured when the kernel changes.
-MEASURED_TRAFFIC_BPP = 836.2
+MEASURED_TRAFFIC_BPP = 778.7
 
 
 def package():
@@ -435,7 +435,7 @@ def main():
             "traffic": MEASURED_TRAFFIC_BPP * n if main_prec == "mixed" else None,
             "traffic_source": "rocprofv3 FETCH_SIZE + WRITE_SIZE passes, copy-calibrated "
                               "(profiles/pmc_traffic_k_force_column1M.md)",
-            "kernel": "k_force_q<mixed, 32> (contact pass, velocity-Verlet integrator fused)",
+            "kernel": "k_force_t<mixed, 32> (contact pass, velocity-Verlet integrator fused)",
             "bytes_per_particle": bpp,
             "avg_launch_ms": avg_ms,
         },
