@@ -742,8 +742,10 @@ static int padded_blocks(long long threads, int block = kBlock)
 //
 // By the count: a small tile is the shorter chain of batches, a large one
 // has fewer half-empty batches and less per-wave work.  The smallest that
-// keeps the waves to what the chip holds at once (256 CUs, 3-4 per SIMD) is
-// the fastest up to there: column of n spheres, mixed, us per pass with tiles
+// keeps the waves to what the chip holds at once (256 CUs; FP64 3 per SIMD,
+// 3072; mixed up to 4) is the fastest up to there, and a few waves past it wait
+// for a whole round (FP64, tiles of 8 / 16: 24,000 14.8 / 16.3; 25,548 17.1 /
+// 15.5; 27,000 18.7 / 16.7; 43,821 21.0 / 17.8): column of n spheres, mixed, us per pass with tiles
 // of 8 / 16 / 32: 20,000 13.5 / 15.5 / 17.8; 50,000 22.0 / 20.0 / 20.8;
 // 200,000 62 / 51 / 46.  From there on 32, and for FP64, whose pass runs at 3
 // waves per SIMD whatever the tile, 64 once both keep every slot busy for many
@@ -760,10 +762,10 @@ static int contact_shape(const ForceArgs &a, bool mixed)
         return 0;
     }();
     if (env) return env;
-    constexpr int kWaves = 3584;
-    if (a.n <= 8 * kWaves) return -8;
-    if (a.n <= 16 * kWaves) return -16;
-    return !mixed && a.n > 112 * kWaves ? -64 : -32;
+    const int waves = mixed ? 3584 : 3072;
+    if (a.n <= 8 * waves) return -8;
+    if (a.n <= 16 * waves) return -16;
+    return !mixed && a.n > 400000 ? -64 : -32;
 }
 
 bool force_can_fuse(const ForceArgs &a) { return a.M.cohesion == CM_OFF; }
