@@ -745,8 +745,8 @@ static int padded_blocks(long long threads, int block = kBlock)
 // keeps the waves to what the chip holds at once (256 CUs; FP64 3 per SIMD,
 // 3072; mixed up to 4) is the fastest up to there, and a few waves past it wait
 // for a whole round (FP64, tiles of 8 / 16: 24,000 14.8 / 16.3; 25,548 17.1 /
-// 15.5; 27,000 18.7 / 16.7; 43,821 21.0 / 17.8): column of n spheres, mixed, us per pass with tiles
-// of 8 / 16 / 32: 20,000 13.5 / 15.5 / 17.8; 50,000 22.0 / 20.0 / 20.8;
+// 15.5; 27,000 18.7 / 16.7; 43,821 21.0 / 17.8): column of n spheres, mixed, us
+// per pass with tiles of 8 / 16 / 32: 20,000 13.5 / 15.5 / 17.8; 50,000 22.0 / 20.0 / 20.8;
 // 200,000 62 / 51 / 46.  From there on 32, and for FP64, whose pass runs at 3
 // waves per SIMD whatever the tile, 64 once both keep every slot busy for many
 // rounds (200,000 55 / 59 with 32 / 64; 500,000 114 / 110; 1M 262 / 248; mixed
