@@ -952,6 +952,7 @@ extern "C" int dem_upload_state(dem_ctx *ctx, int n, const double *x, const doub
             || dev_alloc(ctx, &ctx->stage, c * kStageSlots) || dev_alloc(ctx, &ctx->xn, c)
             || dev_alloc(ctx, &ctx->vn, c) || dev_alloc(ctx, &ctx->wn, c))
             return DEM_ERR_HIP;
+        if (ctx->pwf && dev_alloc(ctx, &ctx->pwf, c)) return DEM_ERR_HIP;   // a plane is observed
         ctx->cap = n;
     }
     ctx->n = n;
