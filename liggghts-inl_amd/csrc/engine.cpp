@@ -115,7 +115,8 @@ struct dem_ctx {
     std::vector<long long> ck_ts;
     std::vector<int> ck_ago;
     char *tape = nullptr;
-    int tape_cap = 0, tape_pos = -1;   // tape_pos >= 0: recording
+    size_t tape_bytes = 0;             // allocated
+    int tape_cap = 0, tape_pos = -1;   // records of the present window; tape_pos >= 0: recording
     std::vector<uint8_t> tape_mask;
     int *adj_rev = nullptr;
     std::vector<const void *> g_key;   // buffers the graph was recorded with
@@ -4204,17 +4205,20 @@ extern "C" int dem_adjoint_backward(dem_ctx *ctx, const double *w_height, const 
     launch_inst_obs(ctx->cstart, ctx->G.nkeys_local, B, sx(ctx), sv(ctx), nullptr, d_cnt, s);
     launch_adj_seed(sw(ctx), w_height ? d_wh : nullptr, d_cnt, lx[0], n, s);
     if (!hip_ok(hipGetLastError(), "seed kernel")) return done(DEM_ERR_HIP);
-    // tape for the longest segment
+    // tape for the longest segment; the record's size follows the particles
+    // and the list of this window
     const size_t tb = state_record_bytes(ctx, false);
-    if (K > ctx->tape_cap) {
+    if (tb * K > ctx->tape_bytes) {
         if (ctx->tape) hipFree(ctx->tape);
         ctx->tape = nullptr;
+        ctx->tape_bytes = 0;
         if (hipMalloc((void **)&ctx->tape, tb * K) != hipSuccess) {
-            ctx->tape_cap = 0;
+            ctx->tape = nullptr;
             return done(fail(ctx, DEM_ERR_NOMEM, "dem_adjoint_backward: out of device memory for the tape"));
         }
-        ctx->tape_cap = K;
+        ctx->tape_bytes = tb * K;
     }
+    ctx->tape_cap = K;
     ctx->tape_mask.assign(K, 0);
     int cur = 0;
     AdjArgs a{};
