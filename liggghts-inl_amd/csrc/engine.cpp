@@ -110,7 +110,7 @@ struct dem_ctx {
     long long setup_ts = -1;           // timestep of the last dem_setup
     bool window = false;               // rebuild steps apply the history mask instead
     int64_t adj_E = 0;                 // list entries of the window
-    int adj_steps = 0, adj_every = 0;
+    int adj_steps = 0, adj_every = 0;  // adj_steps 0: no window, or its particles or list have been replaced
     std::vector<char *> ckpts;         // one per segment start, then the final state
     std::vector<long long> ck_ts;
     std::vector<int> ck_ago;
@@ -957,6 +957,7 @@ extern "C" int dem_upload_state(dem_ctx *ctx, int n, const double *x, const doub
         ctx->cap = n;
     }
     ctx->n = n;
+    ctx->adj_steps = 0;
     ctx->cur = 0;
     ctx->par = 0;
     ctx->maxrad = maxrad;
@@ -1247,6 +1248,7 @@ static int rebuild(dem_ctx *ctx, bool captured = false)
     ctx->lcur = l1;
     ctx->have_list = true;
     ctx->list_valid = true;
+    ctx->adj_steps = 0;
     ctx->ago = 0;
     if (!ctx->meshes.empty() && !ctx->mesh_grids_valid) {
         const int rc = setup_mesh_grids(ctx);
@@ -1711,6 +1713,7 @@ static int append_atoms(dem_ctx *ctx, int m, const double *x, const double *v, c
         return fail(ctx, DEM_ERR_ARG,
                     "dem_append_atoms: not in a batched run, an adjoint window or with an observed plane");
     const int n0 = ctx->n;
+    ctx->adj_steps = 0;
     if ((int64_t)n0 + m > (int64_t)kJMask) return fail(ctx, DEM_ERR_ARG, "dem_append_atoms: too many atoms");
     const int n1 = n0 + m;
     std::vector<double4> hx(m), hv(m), hw(m);
@@ -2860,6 +2863,7 @@ extern "C" int dem_step(dem_ctx *ctx, int nsteps)
             }
             while (st + ctx->g_period <= nsteps - 1 && ctx->ntimestep + ctx->g_period < next_insert_step(ctx)) {
                 HIPCHK(hipGraphLaunch(ctx->gexec, ctx->stream));
+                ctx->adj_steps = 0;   // the period rebuilds
                 ctx->ntimestep += ctx->g_period;
                 st += ctx->g_period;
                 if (ctx->mf.mesh >= 0) {
@@ -3093,6 +3097,7 @@ extern "C" int dem_set_history(dem_ctx *ctx, int64_t count, const int *tag_i, co
         }
     }
     const int l = ctx->lcur;
+    ctx->adj_steps = 0;
     if (ensure_list_cap(ctx, l, count)) return DEM_ERR_NOMEM;
     HIPCHK(hipMemcpy(ctx->nstart[l], cnt.data(), cnt.size() * sizeof(int), hipMemcpyHostToDevice));
     if (count) {
@@ -4095,6 +4100,7 @@ extern "C" int dem_adjoint_forward(dem_ctx *ctx, int nsteps, int checkpoint_ever
     if (!ctx->list_valid || ctx->ntimestep != ctx->setup_ts)
         return fail(ctx, DEM_ERR_ARG, "dem_adjoint_forward: call right after dem_setup");
     sync_enter(ctx);
+    ctx->adj_steps = 0;   // until this forward ends well
     for (char *c : ctx->ckpts) hipFree(c);
     ctx->ckpts.clear();
     ctx->ck_ts.clear();
@@ -4150,7 +4156,8 @@ extern "C" int dem_adjoint_backward(dem_ctx *ctx, const double *w_height, const 
 {
     if (!ctx) return fail(nullptr, DEM_ERR_ARG, "null context");
     if (!grad || ctx->adj_steps < 1 || ctx->ckpts.empty())
-        return fail(ctx, DEM_ERR_ARG, "dem_adjoint_backward: run dem_adjoint_forward first");
+        return fail(ctx, DEM_ERR_ARG, "dem_adjoint_backward: run dem_adjoint_forward first (and neither rebuild nor "
+                                      "replace the particles in between)");
     if (w_wall && ctx->obs_plane < 0)
         return fail(ctx, DEM_ERR_ARG, "dem_adjoint_backward: a wall-force seed needs dem_observe_plane");
     sync_enter(ctx);
