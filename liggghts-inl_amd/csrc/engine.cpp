@@ -213,7 +213,10 @@ struct dem_ctx {
     bool fold = false;
     int fold_par = 0;
     bool cg_fold = false;
-    int check_interval = 0;   // steps between the last two rebuilds that a distance check asked for
+    // steps from a rebuild to the check that asked for the next, the last time
+    // one did; a rebuild forced before (an insertion, a moving mesh) only shows
+    // that it takes at least that long
+    int check_interval = 0;
     double *d_gpart = nullptr, *d_gtot = nullptr;   // partial sums; 4 per op slot
     int ago = 0;
 
@@ -991,6 +994,7 @@ extern "C" int dem_upload_state(dem_ctx *ctx, int n, const double *x, const doub
     // new atoms: massflow side counters not seen yet
     if (ctx->mf.mesh >= 0 && massflow_counters(ctx)) return DEM_ERR_HIP;
     ctx->integ_bit = -1;
+    ctx->check_interval = 0;   // other particles, other speeds
     ctx->have_list = false;
     ctx->list_valid = false;
     ctx->mesh_grids_valid = false;
@@ -2290,6 +2294,8 @@ static int decide(dem_ctx *ctx, int *out)
     *out = 0;
     if (ctx->ntimestep == ctx->next_reneighbor || insert_due(ctx)) {
         *out = 1;
+        // no check has asked in all these steps
+        ctx->check_interval = std::max(ctx->check_interval, ctx->ago);
         return DEM_OK;
     }
     ctx->ago++;
@@ -2307,6 +2313,7 @@ static int decide(dem_ctx *ctx, int *out)
     HIPCHK(hipMemcpyAsync(&h, ctx->d_small + 2, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
     HIPCHK(hipStreamSynchronize(ctx->stream));
     *out = h;
+    if (h) ctx->check_interval = ctx->ago;
     return DEM_OK;
 }
 
@@ -2887,7 +2894,6 @@ extern "C" int dem_step(dem_ctx *ctx, int nsteps)
         // pre_exchange (fix insert) before the build, as Verlet::run
         // (verlet.cpp:304-327)
         if (nflag && !ctx->inserts.empty() && (rc = run_inserts(ctx))) return rc;
-        if (nflag && ctx->p.neigh_check) ctx->check_interval = ctx->ago;
         if (nflag && ctx->n > 0 && (rc = ctx->window ? window_mask(ctx) : rebuild(ctx))) return rc;
         if (!nflag) mesh_trigger(ctx);
         if (ctx->tape_pos >= 0 && (rc = tape_store(ctx, nflag))) return rc;

@@ -57,3 +57,35 @@ def test_runs_equal_single_steps(name, graph):
         assert np.array_equal(p, q)
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize("graph", [False, True])
+def test_runs_between_insertions(graph):
+    """A pour under the distance check into which atoms are inserted every 37
+    steps: rebuilds that an insertion forces lie between those that a check
+    asks for, and each run ends before the next insertion."""
+    eng = load_engine()
+    spec, atoms = eng.workloads.pour_box(n=800, spacing=2.02e-3, jitter=2e-5)
+    hi = spec["box_hi"]
+    spec = dict(spec, neigh_every=1, neigh_check=True, skin=6e-5)
+    ins = dict(seed=15485863, dist_seed=15485867, templates=[dict(type=1, radius=0.9e-3, density=2500.0)],
+               weights=[1.0], region=((0.0, 0.0, 0.6 * hi[2]), tuple(hi)), volumefraction_region=0.2,
+               maxattempt=20, insert_every=37, all_in=True,
+               vel=("uniform", (0.0, 0.0, -0.6), (0.2, 0.2, 0.2)), group_mask=0)
+    a = eng.Simulation(dict(spec, graph=graph), atoms)
+    b = eng.Simulation(spec, atoms)
+    for s in (a, b):
+        s.add_insert_pack(ins)
+        s.setup()
+    for chunk in (150, 2, 148):
+        a.step(chunk)
+        for _ in range(chunk):
+            b.step(1)
+        assert a.n == b.n > 800
+        sa, sb = a.state(), b.state()
+        for k in ("x", "v", "omega", "f", "torque"):
+            assert np.array_equal(sa[k], sb[k]), k
+    for p, q in zip(a.pairs(), b.pairs()):
+        assert np.array_equal(p, q)
+    a.close()
+    b.close()
