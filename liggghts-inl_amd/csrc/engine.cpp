@@ -2463,6 +2463,9 @@ static std::vector<const void *> graph_key(const dem_ctx *ctx)
     k.push_back((const void *)(intptr_t)ctx->n);
     k.push_back((const void *)(intptr_t)(ctx->tune_lanes * 4096 + ctx->tune_block));
     k.push_back((const void *)(intptr_t)ctx->obs_plane);
+    k.push_back((const void *)(intptr_t)ctx->integ_bit);
+    k.push_back(ctx->gmask[0]);
+    k.push_back(ctx->gmask[1]);
     for (const auto &m : ctx->meshes) {
         for (int b = 0; b < 2; b++) {
             k.push_back(m.mstart[b]);
