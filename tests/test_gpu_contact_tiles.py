@@ -7,6 +7,10 @@ overflows into full batches, its entry map (16 per particle) runs out, and the
 first range is empty.  A second run rebuilds on the way, so both ranges are in
 use.  Sizes leave tiles of one, of all but one and of every particle, for
 every tile width and history layout.
+
+Layers passing over each other under a contact distance factor: entries of
+both parts touch and part within reach of the factor, which resets their
+history; with periodic images, two types and frozen spheres.
 """
 import numpy as np
 import pytest
@@ -64,3 +68,59 @@ def test_tiles_at_their_edges(rolling, normal, every):
         if n == 343:
             touching = (np.asarray(o.pairs()[4]) != 0).sum()
             assert touching >= 2 * 3 * 7 * 7 * 6, touching   # every lattice neighbour, both ways
+
+
+def passing(n, rolling, normal, every):
+    """Layers moving in +x and -x by turns, 0.1 um closer than they can pass."""
+    rng = np.random.default_rng(4)
+    side = int(np.ceil(n ** (1 / 3)))
+    g = np.stack(np.meshgrid(*[np.arange(side)] * 3, indexing="ij"), -1).reshape(-1, 3)[:n]
+    odd = g[:, 2] % 2 == 1
+    x = g * [2.05e-3, 2.05e-3, 1.9999e-3] + [-5e-3, 5e-3, 0.9995e-3]
+    x[odd, 0] += rng.uniform(-1e-5, 6e-5, odd.sum())
+    x[:, 0] = np.mod(x[:, 0], 0.03)
+    r = np.full(n, 1e-3)
+    mats = load_engine().workloads._materials(mur=0.1, etar=0.3, ntypes=2)
+    mats["mu"][1, 2] = mats["mu"][2, 1] = 0.2
+    mats["e"][2, 2] = 0.6
+    mats["hysteretic"] = {k: np.full((3, 3), v[1, 1]) for k, v in HYST.items()}
+    spec = dict(box_lo=[0.0] * 3, box_hi=[0.03] * 3, periodic=[1, 0, 0], dt=1e-6, skin=2e-4, cdf=1.05,
+                neigh_every=every, neigh_delay=0, neigh_check=False, rolling=rolling, normal=normal,
+                wall_normal="hertz", materials=mats, planes=[(2, 0.0, 1)], gravity=(0.0, 0.0, -9.81), freeze=True)
+    atoms = dict(x=x, v=np.where(odd, -2.5, 2.5)[:, None] * [1.0, 0.0, 0.0] + rng.uniform(-0.01, 0.01, (n, 3)),
+                 omega=rng.uniform(-20, 20, (n, 3)), radius=r, rmass=4.0 / 3.0 * np.pi * r ** 3 * 2500.0,
+                 type=rng.integers(1, 3, n).astype(np.int32), tag=np.arange(1, n + 1, dtype=np.int32),
+                 freeze=(rng.random(n) < 0.1).astype(np.int32))
+    return spec, atoms
+
+
+@pytest.mark.parametrize("rolling,normal", [("off", "hertz"), ("epsd", "hertz"), ("epsd", "hysteretic/nonlinear1"),
+                                            ("off", "hysteretic/nonlinear2")])
+@pytest.mark.parametrize("every", [1000, 10])
+def test_history_reset_within_the_distance_factor(rolling, normal, every):
+    eng = load_engine()
+    spec, atoms = passing(215, rolling, normal, every)
+    for tile in (-8, -16, -32, -64):
+        for precision in ("fp64", "mixed") if normal == "hertz" else ("fp64",):
+            o = Oracle(spec, atoms)
+            o.add_freeze()
+            o.setup()
+            s = eng.Simulation(spec, atoms, precision=precision)
+            s.set_contact_shape(tile, 0)
+            s.setup()
+            at_build = (o.pairs()[4] != 0).sum()
+            kept = []
+            for _ in range(3):   # most touch, then many have parted, then nearly all
+                s.step(8)
+                o.run(8)
+                kept.append((np.abs(o.pairs()[3]).max(1) > 0).sum())
+                # 24 steps of rounding, as above
+                check_forces(s, o, 1e-9 if precision == "fp64" else 1e-4)
+                check_pairs(s, o, hist_tol=1e-9 if precision == "fp64" else 1e-4)
+                # a reset history is zero, not small
+                gi, gj, gs, gh, gf = s.pairs()
+                zero = {(i, j) for i, j, h in zip(*o.pairs()[:2], o.pairs()[3]) if not h.any()}
+                assert all((i, j) not in zero for i, j, h in zip(gi, gj, gh) if h.any())
+                assert (gf != 0).sum() == (o.pairs()[4] != 0).sum()
+            assert kept[0] > at_build > kept[1] > kept[2]
+            s.close()
