@@ -800,13 +800,18 @@ static void launch_nm(const ForceArgs &a, hipStream_t s)
         default: break;
         }
     }
-    if constexpr (WN == NM_HERTZ)
+    // with hysteretic walls, a rare choice, 8, 16 and 32 are compiled for Hertz
+    // pairs and 32 for hysteretic ones: on few particles a tile of 32 leaves
+    // most of the chip idle (Hertz pairs and nonlinear1 walls, FP64, us per pass
+    // with tiles of 8 / 32: 500 11.3 / 15.2, 8000 12.2 / 15.7, 24,000 14.2 / 16.6)
+    if constexpr (NM == NM_HERTZ || WN == NM_HERTZ)
         switch (shape) {
         case -8: launch_tile<MIXED, NM, WN, 8>(a, B, s); return;
         case -16: launch_tile<MIXED, NM, WN, 16>(a, B, s); return;
-        case -64: launch_tile<MIXED, NM, WN, 64>(a, B, s); return;
         default: break;
         }
+    if constexpr (WN == NM_HERTZ)
+        if (shape == -64) return launch_tile<MIXED, NM, WN, 64>(a, B, s);
     launch_tile<MIXED, NM, WN, 32>(a, B, s);
 }
 

@@ -124,3 +124,37 @@ def test_history_reset_within_the_distance_factor(rolling, normal, every):
                 assert (gf != 0).sum() == (o.pairs()[4] != 0).sum()
             assert kept[0] > at_build > kept[1] > kept[2]
             s.close()
+
+
+@pytest.mark.parametrize("rolling", ["off", "epsd"])
+@pytest.mark.parametrize("wall", ["hysteretic/nonlinear1", "hysteretic/nonlinear2"])
+def test_hertz_pairs_with_hysteretic_walls(wall, rolling):
+    """Every tile that is compiled for this chain, and the width that the
+    particle count gives, with a floor whose history has twelve slots more."""
+    eng = load_engine()
+    for n in (7, 215):
+        spec, atoms = passing(n, rolling, "hertz", 10)
+        spec = dict(spec, wall_normal=wall)
+        for tile in (0, -8, -16, -32):
+            for precision in ("fp64", "mixed"):
+                o = Oracle(spec, atoms)
+                o.add_freeze()
+                o.setup()
+                s = eng.Simulation(spec, atoms, precision=precision)
+                s.set_contact_shape(tile, 0)
+                s.setup()
+                s.step(12)
+                o.run(12)
+                check_forces(s, o, 1e-9 if precision == "fp64" else 1e-4)
+                if n > 7:
+                    check_pairs(s, o, hist_tol=1e-9 if precision == "fp64" else 1e-4)
+                w, ow = s.wall_history(), o.wall_history().reshape(s.wall_history().shape)
+                assert np.abs(w).max() > 0
+                # the slots range over several orders: a scalar against its own
+                # largest, a component (shear, rolling torque) against its vector's
+                top = np.abs(ow).reshape(-1, ow.shape[-1]).max(0)
+                for k in range(12, len(top), 3):
+                    top[k:k + 3] = top[k:k + 3].max()
+                assert (np.abs(w - ow).reshape(-1, ow.shape[-1]).max(0)
+                        <= (1e-9 if precision == "fp64" else 1e-4) * top).all()
+                s.close()
