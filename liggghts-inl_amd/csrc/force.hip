@@ -735,25 +735,62 @@ static int padded_blocks(long long threads, int block = kBlock)
     return (int)((nb + 7) & ~7LL);
 }
 
+// Waves of a chain's tile kernel that the chip holds at once: 256 CUs of four
+// SIMDs, and of a SIMD's 512 registers the law leaves 4 waves (mixed, 128), 3
+// (FP64 Hertz, 142; hysteretic/nonlinear1 in tiles of 8 and 16, 162 to 168) or
+// 2 (hysteretic/nonlinear2, 198 and more).
+static int tile_slots(int nm, int wn, bool mixed)
+{
+    constexpr int simds = 1024;
+    if (nm == NM_HYST2 || wn == NM_HYST2) return 2 * simds;
+    return (mixed && wn == NM_HERTZ ? 4 : 3) * simds;
+}
+
 // Shape of the pass: ForceArgs::lanes/block (set by the autotuner or by
 // hand), else DEM_CONTACT_LANES, else by the particle count.  lanes > 0: lane
-// groups of that width per particle (k_force, Hertz chains); lanes < 0: tiles
-// of -lanes particles per wave (k_force_t).
+// groups of that width per particle (k_force); lanes < 0: tiles of -lanes
+// particles per wave (k_force_t).
 //
 // By the count: a small tile is the shorter chain of batches, a large one
-// has fewer half-empty batches and less per-wave work.  The smallest that
-// keeps the waves to what the chip holds at once (256 CUs; FP64 3 per SIMD,
-// 3072; mixed up to 4) is the fastest up to there, and a few waves past it wait
-// for a whole round (FP64, tiles of 8 / 16: 24,000 14.8 / 16.3; 25,548 17.1 /
-// 15.5; 27,000 18.7 / 16.7; 43,821 21.0 / 17.8): column of n spheres, mixed, us
-// per pass with tiles of 8 / 16 / 32: 20,000 13.5 / 15.5 / 17.8; 50,000 22.0 / 20.0 / 20.8;
-// 200,000 62 / 51 / 46.  From there on 32, and for FP64, whose pass runs at 3
-// waves per SIMD whatever the tile, 64 once both keep every slot busy for many
-// rounds (200,000 55 / 59 with 32 / 64; 500,000 114 / 110; 1M 262 / 248; mixed
-// 231 / 241).
+// has fewer half-empty batches and less per-wave work.  The smallest whose
+// waves fit the slots is the fastest there, and a few waves past them wait
+// for a whole round.  Column of n spheres, us per pass with tiles of
+//              n:    8 /   16        n:    8 /   16        n:   16 /   32
+//   mixed  28,000 14.6 / 14.8   40,000 19.2 / 16.2  100,000 26.0 / 23.5
+//   FP64   24,000 14.2 / 14.9   28,000 18.2 / 15.3   60,000 22.3 / 19.8
+//   nl1    24,000 17.6 / 18.2   28,000 21.3 / 18.5   60,000 27.6 / 25.6
+//   nl2    16,000 15.3 / 15.7   18,000 20.4 / 15.7   40,000 23.9 / 22.5
+// and 16 / 32 on the near side: mixed 60,000 18.4 / 18.9, FP64 48,000 17.8 /
+// 18.5, nl1 48,000 22.6 / 23.6, nl2 32,000 19.7 / 20.5.  From there on 32, and
+// in FP64 64 once both keep every slot busy for many rounds (32 / 64: Hertz
+// 200,000 42.8 / 46.9, 400,000 71.0 / 72.0, 500,000 87.2 / 83.7; nl1 150,000
+// 53.6 / 57.6, 200,000 68.3 / 67.1, 500,000 186 / 170; nl2 150,000 54.3 / 57.3,
+// 200,000 69.4 / 67.4, 500,000 185 / 167; mixed 500,000 73.7 / 81.2).
+static int tile_by_count(int n, int nm, int wn, bool mixed)
+{
+    const int slots = tile_slots(nm, wn, mixed);
+    if (n <= 8 * slots) return -8;
+    if (n <= 16 * slots) return -16;
+    return !mixed && n > 400000 ? -64 : -32;
+}
+
+// Not every shape is compiled for every chain.  Cohesion models: 4 lanes per
+// particle.  Lane groups: Hertz chains with Hertz walls.  Hysteretic walls, a
+// rare choice: tiles of 8, 16 and 32 for Hertz pairs (on few particles a tile
+// of 32 leaves most of the chip idle: nonlinear1 walls, FP64, 8 / 32: 500 11.3 /
+// 15.2, 8000 12.2 / 15.7, 24,000 14.2 / 16.6), 32 for hysteretic ones.
+int force_compiled_shape(int g, const Model &M)
+{
+    if (M.cohesion != CM_OFF) return 4;
+    const bool hp = M.lp.normal == NM_HERTZ, hw = M.lw.normal == NM_HERTZ;
+    if (g > 0) return hp && hw ? g : -32;
+    if (hw || (hp && (g == -8 || g == -16))) return g;
+    return -32;
+}
+
 static int contact_shape(const ForceArgs &a, bool mixed)
 {
-    if (a.lanes) return a.lanes;
+    if (a.lanes) return force_compiled_shape(a.lanes, a.M);
     static const int env = [] {
         const char *s = getenv("DEM_CONTACT_LANES");
         const int g = s ? atoi(s) : 0;
@@ -761,11 +798,8 @@ static int contact_shape(const ForceArgs &a, bool mixed)
             if (g == v) return g;
         return 0;
     }();
-    if (env) return env;
-    const int waves = mixed ? 3584 : 3072;
-    if (a.n <= 8 * waves) return -8;
-    if (a.n <= 16 * waves) return -16;
-    return !mixed && a.n > 400000 ? -64 : -32;
+    if (env) return force_compiled_shape(env, a.M);
+    return force_compiled_shape(tile_by_count(a.n, a.M.lp.normal, a.M.lw.normal, mixed), a.M);
 }
 
 bool force_can_fuse(const ForceArgs &a) { return a.M.cohesion == CM_OFF; }
@@ -781,8 +815,6 @@ static void launch_tile(const ForceArgs &a, int B, hipStream_t s)
     else k_force_t<MIXED, NM, WN, D0 + 3, P><<<nb, B, lds, s>>>(a);
 }
 
-// Hertz pairs with Hertz walls (the common case) take any shape; other model
-// combinations run in tiles.
 template <bool MIXED, int NM, int WN>
 static void launch_nm(const ForceArgs &a, hipStream_t s)
 {
@@ -800,10 +832,6 @@ static void launch_nm(const ForceArgs &a, hipStream_t s)
         default: break;
         }
     }
-    // with hysteretic walls, a rare choice, 8, 16 and 32 are compiled for Hertz
-    // pairs and 32 for hysteretic ones: on few particles a tile of 32 leaves
-    // most of the chip idle (Hertz pairs and nonlinear1 walls, FP64, us per pass
-    // with tiles of 8 / 32: 500 11.3 / 15.2, 8000 12.2 / 15.7, 24,000 14.2 / 16.6)
     if constexpr (NM == NM_HERTZ || WN == NM_HERTZ)
         switch (shape) {
         case -8: launch_tile<MIXED, NM, WN, 8>(a, B, s); return;

@@ -351,6 +351,9 @@ void launch_force_fp64(const ForceArgs &a, hipStream_t s);
 // whether the contact pass of these arguments can integrate (every form
 // without a cohesion model)
 bool force_can_fuse(const ForceArgs &a);
+// the contact pass's shape that runs for this model when g (lanes > 0, tile < 0)
+// is asked for
+int force_compiled_shape(int g, const Model &M);
 void launch_force_mixed(const ForceArgs &a, hipStream_t s);
 // mode: 1 = initial_integrate, 2 = final_integrate, 3 = final then initial
 void launch_integrate(const IntegArgs &a, int mode, hipStream_t s);
