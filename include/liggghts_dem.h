@@ -527,16 +527,19 @@ int dem_instance_observables_noalloc(dem_ctx *ctx, double *out);
  * usual.  The results are bitwise those of stepping without the graph. */
 int dem_use_graph(dem_ctx *ctx, int on);
 /* Autotuner: times the contact pass on the current state for every shape
- * (lane groups of 1..16 lanes per particle, tiles of 8, 16, 32 or 64
- * particles per wave, given as -8..-64) and block size (64..256), in the
- * form the steps run (with the integrator when the pass integrates), and
- * keeps the fastest for this context.  State and history are left
+ * compiled for this context's models (below) and block size (64..256), in
+ * the form the steps run (with the integrator when the pass integrates),
+ * and keeps the fastest for this context.  State and history are left
  * unchanged. */
 int dem_autotune(dem_ctx *ctx, int reps, int *lanes, int *block, double *ms);
-/* Sets the contact pass's shape by hand (lanes per particle 1, 2, 4, 8 or
- * 16, or a contact-queue tile of -8, -16, -32 or -64; block 64, 128 or 256;
- * 0 keeps the default, the -32 queue), e.g. to reuse an earlier autotuner
- * result.  Hertz chains take any shape; others run 4 lanes. */
+/* Sets the contact pass's shape by hand, e.g. to reuse an earlier autotuner
+ * result: lanes per particle 1, 2, 4, 8 or 16, or tiles of 8, 16, 32 or 64
+ * particles per wave given as -8, -16, -32 or -64; block 64, 128 or 256.  0
+ * goes by the particle count, precision and models.  Hertz pairs with Hertz
+ * walls take any shape and hysteretic pairs with Hertz walls any tile; Hertz
+ * pairs with hysteretic walls have tiles of 8, 16 and 32, hysteretic pairs
+ * with hysteretic walls tiles of 32, and other shapes run as tiles of 32
+ * there.  Cohesion models run 4 lanes and 256 threads, whatever is set. */
 int dem_set_contact_shape(dem_ctx *ctx, int lanes, int block);
 
 /* ---- Adjoint window.  No counterpart in the reference (which has no

@@ -4019,7 +4019,6 @@ extern "C" int dem_autotune(dem_ctx *ctx, int reps, int *lanes, int *block, doub
         hipFree(save);
         return fail(ctx, DEM_ERR_HIP, "dem_autotune: copy failed");
     }
-    const bool any_width = ctx->p.normal_model == 0 && ctx->p.wall_normal_model == 0 && ctx->M.cohesion == CM_OFF;
     const int widths[] = {1, 2, 4, 8, 16, -8, -16, -32, -64};   // negative: tiles per wave
     const int blocks[] = {64, 128, 256};
     hipEvent_t e0, e1;
@@ -4028,7 +4027,7 @@ extern "C" int dem_autotune(dem_ctx *ctx, int reps, int *lanes, int *block, doub
     const bool was_timing = ctx->timing;
     ctx->timing = false;
     double best = 1e300;
-    int bl = 4, bb = kBlock;
+    int bl = 0, bb = 0;
     int rc = DEM_OK;
     // time the form the steps run: with the integrator fused when it will
     // be; such a pass writes the new state to the other buffers only, so
@@ -4041,9 +4040,9 @@ extern "C" int dem_autotune(dem_ctx *ctx, int reps, int *lanes, int *block, doub
         return r;
     };
     for (int g : widths) {
-        // chains with a cohesion model have one shape, other non-Hertz chains tiles
-        if (!any_width && (ctx->M.cohesion != CM_OFF ? g != 4 : g > 0)) continue;
+        if (force_compiled_shape(g, ctx->M) != g) continue;   // another shape would run
         for (int b : blocks) {
+            if (ctx->M.cohesion != CM_OFF && b != kBlock) continue;   // one block size there
             ctx->tune_lanes = g;
             ctx->tune_block = b;
             if ((rc = pass())) break;

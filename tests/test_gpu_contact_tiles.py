@@ -158,3 +158,18 @@ def test_hertz_pairs_with_hysteretic_walls(wall, rolling):
                 assert (np.abs(w - ow).reshape(-1, ow.shape[-1]).max(0)
                         <= (1e-9 if precision == "fp64" else 1e-4) * top).all()
                 s.close()
+
+
+@pytest.mark.parametrize("normal,wall,shapes", [
+    ("hertz", "hysteretic/nonlinear1", (-8, -16, -32)), ("hysteretic/nonlinear1", "hertz", (-8, -16, -32, -64)),
+    ("hysteretic/nonlinear2", "hysteretic/nonlinear1", (-32,))])
+def test_autotune_keeps_to_compiled_shapes(normal, wall, shapes):
+    """The shape that the autotuner returns is one that runs for the chain."""
+    eng = load_engine()
+    spec, atoms = passing(215, "epsd", normal, 10)
+    for _ in range(4):
+        s = eng.Simulation(dict(spec, wall_normal=wall), atoms)
+        s.setup()
+        lanes, block, ms = s.autotune(reps=1)
+        assert lanes in shapes and block in (64, 128, 256) and ms > 0.0
+        s.close()

@@ -202,8 +202,8 @@ def test_hopper_short_horizon():
 
 
 def test_hopper_mixed_precision():
-    """The hopper in its stated mixed precision (FP32 pair law in the
-    contact queue, FP64 mesh walls and state): forces within 1e-5 of the
+    """The hopper in its stated mixed precision (FP32 pair law, FP64
+    mesh walls and state): forces within 1e-5 of the
     FP64 oracle from an identical state, and after 40 steps."""
     spec, atoms, o = hopper_state()
     s = sim_from_oracle_mesh(spec, atoms, o, precision="mixed")

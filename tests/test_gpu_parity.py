@@ -209,8 +209,8 @@ SHAPES = ((4, 256), (1, 64), (2, 128), (8, 64), (16, 128), (-8, 256), (-16, 128)
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
 @pytest.mark.parametrize("case", ["pour", "column"])
 def test_contact_shapes_agree(case, precision):
-    """Every contact-pass shape (lane groups 1..16, contact-queue tiles
-    8..64, blocks 64..256) gives the oracle's forces on an identical state,
+    """Every contact-pass shape (lane groups 1..16, tiles of 8..64
+    particles, blocks 64..256) gives the oracle's forces on an identical state,
     in FP64 (1e-12: the shapes differ only in the order each particle's
     contacts are summed) and in mixed precision (1e-5, the FP32 law)."""
     spec, atoms, o = pour_state() if case == "pour" else column_state(n=6000, steps=40)
