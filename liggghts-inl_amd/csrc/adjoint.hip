@@ -97,7 +97,8 @@ __device__ inline LawP law_params(const double *mat, int it, int jt)
 // order, own before reverse, from LDS: the sums a single thread walking the
 // row would form.  The particle's first lane goes on to the planes.
 // One reverse sweep of the law is a chain of several hundred FP64 operations on
-// 256 registers: the chain and two waves per SIMD bound the pass.  With a
+// 256 registers and two spilled ones: the chain and two waves per SIMD bound the
+// pass.  With a
 // thread per particle, 22,793 spheres filled 90 blocks and a pass lasted as
 // long as the longest row's two sweeps per contact: 120 us, 60 us now (the
 // whole gradient, 400 steps, 77.5 -> 51 ms).  8 lanes give the same there and

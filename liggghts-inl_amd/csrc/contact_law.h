@@ -46,8 +46,8 @@ struct NormalOut {
 // correctly rounded operations; root4 adds the first-order rest of its two
 // roots (from their residuals, exact in an fma) to the rounded ones: largest
 // error 0.50 ulp (the pow 1.00) over 1e-13..20.  Contact pass of a 100,000-
-// sphere hysteretic/nonlinear1 column: 70 -> 55 us (registers 218 -> 170, two
-// waves per SIMD in both).
+// sphere hysteretic/nonlinear1 column, tiles of 32: 70 -> 55 us (registers 218 ->
+// 170, two waves per SIMD in both; tiles of 8 and 16 take 166 and 168, three).
 template <bool INVERSE>
 __device__ inline double root4(double z)
 {

@@ -368,13 +368,14 @@ __global__ void __launch_bounds__(kBlock) k_force(ForceArgs a)
 //
 // What bounds it: the latency of its chain of gathers at 4 (mixed) or 3
 // (FP64) waves per SIMD, which the 128 / 142 registers of the law allow, with
-// 48 % of the issue slots taken by VALU.  Of the 700 B per particle of HBM
-// traffic 195 + 195 are histories; with rows of touching and other partners
-// mixed (whole rows one after the other) it was 836 B, and every entry went
-// through the test and a queue.  1M-sphere column: 276 -> 231 us mixed, 282 ->
-// 242 FP64.  Slower here: histories and state through LDS in whole lines (249
-// to 270 us), the first batch fetched ahead of the test (256, one wave per
-// SIMD fewer), tiles trimmed so that their batches fill (236).
+// 48 % of the issue slots taken by VALU.  1M-sphere column: 276 -> 231 us mixed,
+// 282 -> 242 FP64, where every entry of whole rows, one after the other, went
+// through the test and a queue.  HBM traffic there (4.52 contacts and 7.58
+// partners per particle, 652 B that the pass cannot do without) 836 -> 779 B per
+// particle, of which 217 + 217 are histories.  Slower here: histories and state
+// through LDS in whole lines (249 to 270 us), the first batch fetched ahead of
+// the test (256, one wave per SIMD fewer), tiles trimmed so that their batches
+// fill (236).
 constexpr int kQueue = 192;   // 63 waiting and the 128 of one test
 
 template <int P, typename OutT>
