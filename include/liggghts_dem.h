@@ -523,8 +523,10 @@ int dem_instance_observables(dem_ctx *ctx, double *out);
 int dem_instance_observables_noalloc(dem_ctx *ctx, double *out);
 /* Step with a recorded HIP graph of two rebuild periods when every rebuild
  * falls on a fixed step (neigh_modify check no, mesh walls only if none
- * moves, no bonds, no setforce/aveforce, timing off); other steps run as
- * usual.  The results are bitwise those of stepping without the graph. */
+ * moves, no bonds, no setforce/aveforce, timing off), or of 16 steps with
+ * their distance checks (check yes, every 1, delay 0; no setforce/aveforce
+ * or fix move); other steps run as usual.  The results are bitwise those of
+ * stepping without the graph. */
 int dem_use_graph(dem_ctx *ctx, int on);
 /* Autotuner: times the contact pass on the current state for every shape
  * compiled for this context's models (below) and block size (64..256), in
@@ -556,7 +558,8 @@ int dem_adjoint_forward(dem_ctx *ctx, int nsteps, int checkpoint_every);
  * observed plane on instance b), at the window's last step (either weight
  * array may be NULL).  grad[4b..4b+3] = dJ/d(Yeff, Geff, betaeff, mu) of
  * instance b, summed over its type pairs.  The context is left at the
- * window's final state. */
+ * window's final state.  The window lasts until its particles or its list
+ * are replaced (upload, insertion, set-up, rebuild, a later forward). */
 int dem_adjoint_backward(dem_ctx *ctx, const double *w_height, const double *w_wall, double *grad);
 
 #ifdef __cplusplus
